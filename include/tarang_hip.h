@@ -241,11 +241,10 @@ typedef struct {
     int dtype;
     int timestepper;
     double b_bottom, b_top;  /* Dirichlet values b(z=0), b(z=Lz) (the test problem: Lz, 0) */
-    int refine_sweeps;       /* 0, 1 or 2 sweeps of x += A^-1 (y - A x) per implicit solve, with the
-                                residual y - A x formed in FP64 from the structured tau systems */
-    int split_inverse;       /* FP32 state only: 1 stores every inverse entry as an FP32 value plus
-                                an 8-bit remainder (2^-32 relative instead of 2^-24, 5 bytes per
-                                entry instead of 4); 0 plain FP32 inverses */
+    int refine_sweeps;       /* 0, 1 or 2, checked and otherwise without effect: the implicit solves are
+                                direct, in FP64 arithmetic, and leave nothing to refine */
+    int split_inverse;       /* 0 or 1 (1: FP32 state only), checked and otherwise without effect: no
+                                inverse is stored */
 } tarang_chan_desc;
 
 #define TARANG_CHAN_P 0

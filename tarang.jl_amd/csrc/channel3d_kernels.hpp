@@ -206,277 +206,8 @@ __global__ __launch_bounds__(NT) void k3_yfwd(const cplx<T>* __restrict__ H, Ch3
     }
 }
 
-// ---------------------------------------------------------------------------
-// Per-mode systems.  With ux = i ux~, uy = i uy~ (E3x, E3y rows times -i) and the
-// horizontal velocity rotated onto k_h = (kx, ky):
-//   u~par = (kx ux~ + ky uy~)/|k_h|,  u~perp = (-ky ux~ + kx uy~)/|k_h|   (x, y at k_h = 0)
-// every mode splits into: the b system (kappa), the perp system (nu, walls 0) and
-// the 2-D u-p system with kx -> |k_h|, each in two parity groups.  The systems
-// depend on |k_h|^2 only; modes share the inverses of their key.
-// ---------------------------------------------------------------------------
-struct Ch3Sys {
-    int N, nkeys;
-    size_t sb, su;
-    const double* kh;   // [nkeys], key 0 is kx = ky = 0
-    double sz, kappa, nu, c, area, Lz;
-};
-
-// grid (2 nkeys, 3): blockIdx.x = 2 key + g; y = 0 b, 1 u-p, 2 perp
-static __global__ void k3_assemble(Ch3Sys s, double* Ab, double* Aup, double* Ap) {
-    const int w = blockIdx.x, key = w >> 1, g = w & 1;
-    const double kh = s.kh[key];
-    if (blockIdx.y == 1) {
-        const int n = chu_size(s.N, g, key);
-        double* A = Aup + (size_t)w * s.su;
-        for (size_t idx = threadIdx.x; idx < (size_t)n * n; idx += blockDim.x)
-            A[idx] = chu_entry_kh(s.N, g, key == 0, kh, s.nu, s.c, s.sz, s.area, s.Lz, (int)(idx % n),
-                                  (int)(idx / n));
-    } else {
-        const int n = chb_size(s.N, g);
-        const double diff = blockIdx.y == 0 ? s.kappa : s.nu;
-        double* A = (blockIdx.y == 0 ? Ab : Ap) + (size_t)w * s.sb;
-        for (size_t idx = threadIdx.x; idx < (size_t)n * n; idx += blockDim.x)
-            A[idx] = chb_entry_kh(s.N, g, kh, diff, s.c, s.sz, (int)(idx % n), (int)(idx / n));
-    }
-}
-
-struct Ch3SolveArgs {
-    // b-system inverses, stride sb per (key, parity): FP64 column-major (ld = n), or FP32
-    // packed by pk_index
-    const void* Ib;
-    const void* Ip;     // perp-system inverses, stride sb
-    const void* Iu;     // u-p-system inverses, stride su
-    // 8-bit remainders of the FP32 inverses (split inverses), same offsets; null otherwise
-    const signed char *Iblo, *Iplo, *Iulo;
-    const int4* chunks; // [nchunks] (key, g, first, count): modes[first .. first + count), count <= 8
-    const int* modes;   // modes grouped by key
-    const double* rot;  // [2 nmodes] (cos, sin) of the k_h direction per mode
-    int N;
-    size_t sb, su;
-    double c;
-    const double2* bcv;  // [2 m + w]: b on wall w (0: z=0, 1: z=Lz) at mode m (unnormalised 2-D rfft)
-    // iterative refinement: sweeps of x += A^-1 (y - A x) with the residual formed in FP64 from
-    // the structured systems (chb_residual / chu_residual); 0 = none
-    int sweeps;
-    const double* kh;  // [nkeys] |k_h| per key
-    double kappa, nu, sz, area, Lz;
-};
-
 // 3-D tau slots: 0 tau_p, 1 tau_b1, 2 tau_b2, 3 tau_u1x, 4 tau_u1y, 5 tau_u1z, 6 tau_u2x, 7 tau_u2y, 8 tau_u2z
 constexpr int kCh3TauStride = 9;
-constexpr int kCh3ChunkModes = 8;  // modes per workgroup: 16 real right-hand sides
-
-__host__ __device__ inline int round16(int n) { return (n + 15) & ~15; }
-
-// k3_solve's small size class for 256-thread workgroups (4 waves)
-inline bool ch3_solve_small(int nb_max, int nu_max) {
-    return (nu_max + 15) / 16 <= 16 && (nb_max + 15) / 16 <= 8;
-}
-
-// right-hand sides, and with refinement a second block set for the solutions
-__host__ __device__ inline size_t ch3_solve_lds_doubles(int N, bool refine = false) {
-    return (size_t)kYS * (2 * round16(chb_size(N, 0)) + round16(chu_size(N, 0, 0))) * (refine ? 2 : 1);
-}
-
-// A^-1 Y for one system: FP64 inverses column-major; FP32 inverses packed, with their
-// 8-bit remainders when SPLIT
-template <int MT, typename T, bool SPLIT, int D = 2>
-__device__ inline void ch3_apply(const void* I, const signed char* Ilo, size_t off, int n, const double* Y,
-                                 dbl4 (&acc)[MT], int wave, int nw, int wave0, bool accumulate = false) {
-    if constexpr (sizeof(T) == 4)
-        mfma_apply_pk<MT, SPLIT, D>(static_cast<const float*>(I) + off, SPLIT ? Ilo + off : nullptr, n, Y, acc, wave,
-                                    nw, wave0, accumulate);
-    else
-        mfma_apply<MT, double, D>(static_cast<const double*>(I) + off, n, Y, acc, wave, nw, wave0, accumulate);
-}
-
-// Workgroup = (|k_h| key, parity g, up to 8 modes of that key).  Right-hand sides of
-// the modes are the columns of 16-column blocks in LDS (column 2 j = real, 2 j + 1 =
-// imaginary part of mode j); every system is applied as X = A^-1 Y on the FP64 matrix
-// cores, so each inverse is read once per chunk.  The inverses are stored in the state
-// precision T (formed in FP64; rounding them to FP32 costs the same relative error as
-// rounding the right-hand side to FP32), the products accumulate in FP64.  Order: b system of parity h = g^1
-// and the perp system of parity g together, then the u-p system of parity g (its
-// E3z rows take + c b), then the un-rotation of the parity-g horizontal velocity.
-// SMALL: at most 4 u-p and 2 b/perp tiles per wave (nu <= 256, nb <= 128 with NT = 256),
-// which keeps the accumulators and load buffers of a 3-workgroup-per-CU launch in
-// registers; the larger FP32 class (wider packed-load buffers) runs 2 workgroups per CU.
-// D: depth of the inverse-load ring (D - 1 batches of entries in flight per wave)
-template <typename T, int NT, bool REFINE = false, bool SPLIT = false, bool SMALL = false, int D = 2>
-__global__ __launch_bounds__(NT, REFINE ? 1 : (SMALL || sizeof(T) == 8 ? 768 : 512) / NT) void k3_solve(Ch3SolveArgs s, const cplx<T>* __restrict__ R1,
-                                               const cplx<T>* __restrict__ R2, const cplx<T>* __restrict__ R3x,
-                                               const cplx<T>* __restrict__ R3y, const cplx<T>* __restrict__ R3z,
-                                               cplx<T>* P, cplx<T>* B, cplx<T>* UX, cplx<T>* UY, cplx<T>* UZ,
-                                               cplx<T>* taus) {
-    static_assert(NT == 256 || NT == 512, "four or eight wavefronts per workgroup");
-    static_assert(!SPLIT || sizeof(T) == 4, "split inverses belong to the FP32 state");
-    constexpr int MTB = SMALL || NT == 512 ? 2 : 3, MTU = SMALL || NT == 512 ? 4 : 7;  // tiles per wave (nz <= 256)
-    extern __shared__ unsigned char smem_raw[];
-    __shared__ int smode[kCh3ChunkModes];
-    __shared__ double srot[2 * kCh3ChunkModes];
-    const int4 ch = s.chunks[blockIdx.x];
-    const int key = ch.x, g = ch.y, first = ch.z, cnt = ch.w;
-    if (cnt <= 0) return;  // padding entry: the whole workgroup leaves before any barrier
-    const int N = s.N, h = g ^ 1, PL = (N - 1) & 1;
-    const int ng = npar(N, g), nh = npar(N, h);
-    const int nb = nh + 1, np = ng + 1, nu = chu_size(N, g, key);  // key 0 is kx = ky = 0 only
-    double* Yb = reinterpret_cast<double*>(smem_raw);  // [round16(nb)][kYS]
-    double* Yp = Yb + kYS * round16(nb);                // [round16(np)][kYS]
-    double* Yu = Yp + kYS * round16(np);                // [round16(nu)][kYS]
-    const int ytot = kYS * (round16(nb) + round16(np) + round16(nu));
-    // solutions: in place over the right-hand sides, or (refinement) in blocks of their own
-    const int sweeps = REFINE ? s.sweeps : 0;  // the LDS holds the solution blocks only when refining
-    double* Xb = sweeps ? Yb + ytot : Yb;
-    double* Xp = sweeps ? Yp + ytot : Yp;
-    double* Xu = sweeps ? Yu + ytot : Yu;
-    if (threadIdx.x < kCh3ChunkModes) {
-        const int j = threadIdx.x;
-        const int q = j < cnt ? s.modes[first + j] : -1;
-        smode[j] = q;
-        srot[2 * j] = q >= 0 ? s.rot[2 * q] : 1.0;
-        srot[2 * j + 1] = q >= 0 ? s.rot[2 * q + 1] : 0.0;
-    }
-    for (int idx = threadIdx.x; idx < (sweeps ? 2 : 1) * ytot; idx += NT) Yb[idx] = 0.0;
-    __syncthreads();
-    // ---- right-hand sides ----
-    for (int idx = threadIdx.x; idx < cnt * nh; idx += NT) {
-        const int j = idx / nh, i = idx - j * nh;
-        const size_t base = (size_t)smode[j] * N;
-        const cplx<T> r = R2[base + 2 * i + h], rz = R3z[base + 2 * i + h];
-        Yb[i * kYS + 2 * j] = (double)r.x;
-        Yb[i * kYS + 2 * j + 1] = (double)r.y;
-        Yu[(2 * ng + i) * kYS + 2 * j] = (double)rz.x;
-        Yu[(2 * ng + i) * kYS + 2 * j + 1] = (double)rz.y;
-    }
-    for (int idx = threadIdx.x; idx < cnt * ng; idx += NT) {
-        const int j = idx / ng, i = idx - j * ng;
-        const size_t base = (size_t)smode[j] * N;
-        const double cr = srot[2 * j], sr = srot[2 * j + 1];
-        const cplx<T> rx = R3x[base + 2 * i + g], ry = R3y[base + 2 * i + g], r1 = R1[base + 2 * i + g];
-        const double ex_re = (double)rx.y, ex_im = -(double)rx.x;  // rows -i E3x, -i E3y
-        const double ey_re = (double)ry.y, ey_im = -(double)ry.x;
-        Yp[i * kYS + 2 * j] = -sr * ex_re + cr * ey_re;  // perp: -sin E3x + cos E3y
-        Yp[i * kYS + 2 * j + 1] = -sr * ex_im + cr * ey_im;
-        Yu[i * kYS + 2 * j] = cr * ex_re + sr * ey_re;  // par: cos E3x + sin E3y
-        Yu[i * kYS + 2 * j + 1] = cr * ex_im + sr * ey_im;
-        Yu[(ng + i) * kYS + 2 * j] = (double)r1.x;
-        Yu[(ng + i) * kYS + 2 * j + 1] = (double)r1.y;
-    }
-    for (int j = threadIdx.x; j < cnt; j += NT) {  // wall rows of b: half-sum / half-difference per mode
-        const double2 g0 = s.bcv[2 * (size_t)smode[j]], g1 = s.bcv[2 * (size_t)smode[j] + 1];
-        Yb[nh * kYS + 2 * j] = s.c * (h == 0 ? 0.5 * (g1.x + g0.x) : 0.5 * (g1.x - g0.x));
-        Yb[nh * kYS + 2 * j + 1] = s.c * (h == 0 ? 0.5 * (g1.y + g0.y) : 0.5 * (g1.y - g0.y));
-    }
-    __syncthreads();
-    // ---- b (parity h) and perp (parity g) systems ----
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = NT / 64, w0p = ((nb + 15) >> 4) % nw;
-    const double kh = s.kh[key];
-    const size_t ob = (size_t)(2 * key + h) * s.sb, op = (size_t)(2 * key + g) * s.sb;
-    if constexpr (!REFINE) {
-        // the b system on the first half of the waves, the perp system on the second: each
-        // wave runs one load pipeline, with twice the tiles in flight
-        constexpr int MTH = 2 * MTB;
-        const int half = nw / 2;
-        const bool isb = wave < half;  // wave-uniform
-        dbl4 acc[MTH];
-        if (isb) ch3_apply<MTH, T, SPLIT, D>(s.Ib, s.Iblo, ob, nb, Yb, acc, wave, half, 0);
-        else ch3_apply<MTH, T, SPLIT, D>(s.Ip, s.Iplo, op, np, Yp, acc, wave - half, half, 0);
-        __syncthreads();  // the solutions overwrite the right-hand sides every wave of the group reads
-        if (isb) mfma_store<MTH>(acc, nb, Xb, wave, half, 0);
-        else mfma_store<MTH>(acc, np, Xp, wave - half, half, 0);
-    } else {
-        dbl4 ab[MTB], ap[MTB];
-        ch3_apply<MTB, T, SPLIT, D>(s.Ib, s.Iblo, ob, nb, Yb, ab, wave, nw, 0);
-        ch3_apply<MTB, T, SPLIT, D>(s.Ip, s.Iplo, op, np, Yp, ap, wave, nw, w0p);
-        __syncthreads();
-        mfma_store<MTB>(ab, nb, Xb, wave, nw, 0);
-        mfma_store<MTB>(ap, np, Xp, wave, nw, w0p);
-        for (int sw = 0; sw < sweeps; ++sw) {
-            __syncthreads();
-            if (threadIdx.x < 16) chb_residual(N, h, kh, s.kappa, s.c, s.sz, Yb, Xb, kYS, 1, threadIdx.x);
-            else if (threadIdx.x < 32) chb_residual(N, g, kh, s.nu, s.c, s.sz, Yp, Xp, kYS, 1, threadIdx.x - 16);
-            __syncthreads();
-            ch3_apply<MTB, T, SPLIT, D>(s.Ib, s.Iblo, ob, nb, Xb, ab, wave, nw, 0, true);  // x += A^-1 r
-            ch3_apply<MTB, T, SPLIT, D>(s.Ip, s.Iplo, op, np, Xp, ap, wave, nw, w0p, true);
-            __syncthreads();
-            mfma_store<MTB>(ab, nb, Xb, wave, nw, 0);
-            mfma_store<MTB>(ap, np, Xp, wave, nw, w0p);
-        }
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < cnt * nh; idx += NT) {
-        const int j = idx / nh, i = idx - j * nh;
-        const double bre = Xb[i * kYS + 2 * j], bim = Xb[i * kYS + 2 * j + 1];
-        Yu[(2 * ng + i) * kYS + 2 * j] += s.c * bre;
-        Yu[(2 * ng + i) * kYS + 2 * j + 1] += s.c * bim;
-        B[(size_t)smode[j] * N + 2 * i + h] = cplx<T>{T(bre), T(bim)};
-    }
-    if (threadIdx.x < cnt) {
-        const int j = threadIdx.x;
-        taus[(size_t)smode[j] * kCh3TauStride + (h == (PL ^ 1) ? 1 : 2)] =
-            cplx<T>{T(Xb[nh * kYS + 2 * j]), T(Xb[nh * kYS + 2 * j + 1])};
-    }
-    __syncthreads();
-    // ---- u-p system of parity g ----
-    {
-        const size_t ou = (size_t)(2 * key + g) * s.su;
-        dbl4 au[MTU];
-        ch3_apply<MTU, T, SPLIT, D>(s.Iu, s.Iulo, ou, nu, Yu, au, wave, nw, 0);
-        __syncthreads();
-        mfma_store<MTU>(au, nu, Xu, wave, nw, 0);
-        for (int sw = 0; REFINE && sw < sweeps; ++sw) {
-            __syncthreads();
-            if (threadIdx.x < 16)
-                chu_residual(N, g, key == 0, kh, s.nu, s.c, s.sz, s.area, s.Lz, Yu, Xu, kYS, 1, threadIdx.x);
-            __syncthreads();
-            ch3_apply<MTU, T, SPLIT, D>(s.Iu, s.Iulo, ou, nu, Xu, au, wave, nw, 0, true);  // x += A^-1 r
-            __syncthreads();
-            mfma_store<MTU>(au, nu, Xu, wave, nw, 0);
-        }
-    }
-    __syncthreads();
-    // un-rotate: u~x = cos par - sin perp, u~y = sin par + cos perp; u = i u~
-    for (int idx = threadIdx.x; idx < cnt * ng; idx += NT) {
-        const int j = idx / ng, i = idx - j * ng;
-        const size_t o = (size_t)smode[j] * N + 2 * i + g;
-        const double cr = srot[2 * j], sr = srot[2 * j + 1];
-        const double par_re = Xu[i * kYS + 2 * j], par_im = Xu[i * kYS + 2 * j + 1];
-        const double pe_re = Xp[i * kYS + 2 * j], pe_im = Xp[i * kYS + 2 * j + 1];
-        const double tx_re = cr * par_re - sr * pe_re, tx_im = cr * par_im - sr * pe_im;
-        const double ty_re = sr * par_re + cr * pe_re, ty_im = sr * par_im + cr * pe_im;
-        UX[o] = cplx<T>{T(-tx_im), T(tx_re)};
-        UY[o] = cplx<T>{T(-ty_im), T(ty_re)};
-        P[o] = cplx<T>{T(Xu[(ng + i) * kYS + 2 * j]), T(Xu[(ng + i) * kYS + 2 * j + 1])};
-    }
-    for (int idx = threadIdx.x; idx < cnt * nh; idx += NT) {
-        const int j = idx / nh, i = idx - j * nh;
-        UZ[(size_t)smode[j] * N + 2 * i + h] =
-            cplx<T>{T(Xu[(2 * ng + i) * kYS + 2 * j]), T(Xu[(2 * ng + i) * kYS + 2 * j + 1])};
-    }
-    if (threadIdx.x < cnt) {
-        const int j = threadIdx.x, mode = smode[j];
-        const double cr = srot[2 * j], sr = srot[2 * j + 1];
-        const double pt_re = Xp[ng * kYS + 2 * j], pt_im = Xp[ng * kYS + 2 * j + 1];  // perp-system tau
-        cplx<T>* tm = taus + (size_t)mode * kCh3TauStride;
-        const int t0 = 2 * ng + nh;
-        for (int t = 0; t < nu - t0; ++t) {
-            const int slot = chu_tau_slot(N, g, t);  // 2-D slots: 0 p, 3 u1x, 4 u1z, 5 u2x, 6 u2z
-            const double re = Xu[(t0 + t) * kYS + 2 * j], im = Xu[(t0 + t) * kYS + 2 * j + 1];
-            if (slot == 0) {
-                tm[0] = cplx<T>{T(re), T(im)};
-            } else if (slot == 4 || slot == 6) {
-                tm[slot == 4 ? 5 : 8] = cplx<T>{T(re), T(im)};
-            } else {  // horizontal lift tau: par from this system, perp from the perp system (same lift)
-                const double tx_re = cr * re - sr * pt_re, tx_im = cr * im - sr * pt_im;
-                const double ty_re = sr * re + cr * pt_re, ty_im = sr * im + cr * pt_im;
-                const int sx = slot == 3 ? 3 : 6;
-                tm[sx] = cplx<T>{T(-tx_im), T(tx_re)};
-                tm[sx + 1] = cplx<T>{T(-ty_im), T(ty_re)};
-            }
-        }
-        if (mode != 0 && g == 0) tm[0] = cplx<T>{T(0), T(0)};
-    }
-}
 
 // Multistep right-hand side with the grid round trip of the state (Hermitian part
 // of the kx = 0 and kx = Nx/2 lines), scaled by 1/a0; histories replaced in place.

@@ -3,8 +3,7 @@
 // Step (src/core/timesteppers/step_subproblem_multistep.jl:197-420, _sbdf2_coefs :544-552):
 //   F_n = F(P(x_n)) (z-backward, padded y and x passes, z-forward), M P(x_n)
 //   rhs = (c1 F_n + c2 F_{n-1} - a1 M P(x_n) - a2 M P(x_{n-1})) / a0, BC rows c ALG
-//   x_{n+1} = (M + L/a0)^-1 rhs  per mode: three parity-split systems per parity, whose
-//   explicit inverses (formed in FP64 per |k_h|^2 key) are applied to 8-mode chunks
+//   x_{n+1} = (M + L/a0)^-1 rhs  per mode: direct FP64 line solves (tau_solve.hpp)
 // SBDF1 on the first step after create / set_field, SBDF2 (w = dt/dt_prev) after.
 #include <algorithm>
 #include <array>
@@ -46,8 +45,8 @@ void Channel3Solver::validate(const Channel3Desc& d) {
                "3-D channel solver: ChebyshevT size " + std::to_string(d.nz) + " unsupported (4..256)");
     TG_REQUIRE(d.refine_sweeps >= 0 && d.refine_sweeps <= 2, kErrInvalid,
                "3-D channel solver: refine_sweeps must be 0, 1 or 2");
-    TG_REQUIRE(d.refine_sweeps == 0 || ch3_solve_lds_doubles(d.nz, true) * sizeof(double) <= 160 * 1024, kErrInvalid,
-               "3-D channel solver: refinement sweeps need nz <= 208 (LDS of the solve)");
+    TG_REQUIRE(d.refine_sweeps == 0 || d.nz <= 208, kErrInvalid,
+               "3-D channel solver: refinement sweeps need nz <= 208");
     TG_REQUIRE(d.split_inverse == 0 || (d.split_inverse == 1 && d.dtype == kF32), kErrInvalid,
                "3-D channel solver: split_inverse is 0, or 1 with an FP32 state");
     TG_REQUIRE(d.Lx > 0 && d.Ly > 0 && d.Lz > 0 && d.dt > 0, kErrInvalid,
@@ -60,8 +59,6 @@ Channel3Solver::Channel3Solver(Context* ctx, const Channel3Desc& d) : ctx_(ctx),
     nmodes_ = nxh_ * d.ny;
     mx_ = padded_len(d.nx);
     my_ = padded_len(d.ny);
-    nb_max_ = chb_size(d.nz, 0);
-    nu_max_ = chu_size(d.nz, 0, 0);
     dt_prev_ = d.dt;
     ctx_->activate();
     hipStream_t s = ctx_->stream;
@@ -138,68 +135,20 @@ Channel3Solver::Channel3Solver(Context* ctx, const Channel3Desc& d) : ctx_(ctx),
     }
     // the only mode with key 0 is kx = ky = 0 (integer keys), so the tau_p system is key 0
     nkeys_ = (int)khv.size();
-    // chunks of up to 8 modes of one key, one workgroup per (chunk, parity); the chunks of a
-    // (key, parity) sit kXcds positions apart in the launch order, so that consecutive
-    // workgroups of one XCD share the key's inverses in that XCD's L2
-    std::vector<int> modes(nmodes_);
-    for (int q = 0; q < nmodes_; ++q) modes[q] = q;
-    std::stable_sort(modes.begin(), modes.end(), [&](int a, int b) { return key[a] < key[b]; });
-    key_count_.assign(nkeys_, 0);
-    for (int q = 0; q < nmodes_; ++q) key_count_[key[q]] += 1;
-    constexpr int kXcds = 8;
-    std::vector<std::vector<std::array<int, 4>>> bucket(kXcds);
-    {
-        std::vector<int> start(nkeys_ + 1, 0);
-        for (int k = 0; k < nkeys_; ++k) start[k + 1] = start[k] + key_count_[k];
-        for (int k = 0; k < nkeys_; ++k)
-            for (int g = 0; g < 2; ++g) {
-                size_t best = 0;
-                for (int x = 1; x < kXcds; ++x)
-                    if (bucket[x].size() < bucket[best].size()) best = x;
-                for (int f = start[k]; f < start[k + 1]; f += kCh3ChunkModes)
-                    bucket[best].push_back({k, g, f, std::min(kCh3ChunkModes, start[k + 1] - f)});
-            }
-    }
-    size_t depth = 0;
-    for (auto& b : bucket) depth = std::max(depth, b.size());
-    std::vector<int> chunks(4 * kXcds * depth, 0);  // padding entries have count 0
-    for (size_t p = 0; p < kXcds * depth; ++p) {
-        const auto& b = bucket[p % kXcds];
-        if (p / kXcds < b.size())
-            for (int e = 0; e < 4; ++e) chunks[4 * p + e] = b[p / kXcds][e];
-    }
-    nchunks_ = (int)(kXcds * depth);
+    // modes sorted by key: neighbouring waves of the solve read the same key's table
+    std::vector<int2> modes(nmodes_);
+    for (int q = 0; q < nmodes_; ++q) modes[q] = int2{q, key[q]};
+    std::stable_sort(modes.begin(), modes.end(), [](const int2& a, const int2& b) { return a.y < b.y; });
+    kh_max_ = *std::max_element(khv.begin(), khv.end());
     auto up = [&](DevBuf& b, const void* h, size_t bytes) {
         b = DevBuf(ctx_, bytes);
         TG_HIP(hipMemcpyAsync(b.ptr, h, bytes, hipMemcpyHostToDevice, s));
         TG_HIP(hipStreamSynchronize(s));
     };
     up(kh_, khv.data(), khv.size() * sizeof(double));
-    up(modes_, modes.data(), modes.size() * sizeof(int));
-    up(chunks_, chunks.data(), chunks.size() * sizeof(int));
+    up(modes_, modes.data(), modes.size() * sizeof(int2));
     up(rot_, rot.data(), rot.size() * sizeof(double));
-    {
-        // inverses in the state precision; FP32 ones packed for 16-byte loads, their padding
-        // columns zero (the factorisations rewrite only the entries of each system)
-        const bool pack = d.dtype == kF32;
-        const size_t ib = dtype_size((DType)d.dtype);
-        sb_ = inverse_stride(nb_max_, pack);
-        su_ = inverse_stride(nu_max_, pack);
-        auto zeroed = [&](size_t bytes) {
-            DevBuf b(ctx_, bytes);
-            TG_HIP(hipMemsetAsync(b.ptr, 0, bytes, s));
-            return b;
-        };
-        Ib_ = zeroed((size_t)2 * nkeys_ * sb_ * ib);
-        Ip_ = zeroed((size_t)2 * nkeys_ * sb_ * ib);
-        Iu_ = zeroed((size_t)2 * nkeys_ * su_ * ib);
-        if (d.split_inverse) {
-            Iblo_ = zeroed((size_t)2 * nkeys_ * sb_);
-            Iplo_ = zeroed((size_t)2 * nkeys_ * sb_);
-            Iulo_ = zeroed((size_t)2 * nkeys_ * su_);
-        }
-    }
-    info_ = DevBuf(ctx_, (size_t)6 * nkeys_ * sizeof(int));
+    tab_tau_ = DevBuf(ctx_, tau_table_doubles(tau_shape(d.nz, true), nkeys_) * sizeof(double));
     {
         const auto bcv = constant_wall_values((size_t)nmodes_, (double)d.nx * d.ny, d.b_bottom, d.b_top);
         bcv_ = DevBuf(ctx_, bcv.size() * sizeof(double2));
@@ -221,7 +170,7 @@ void Channel3Solver::set_tuning(const Chan3Tuning& t) {
     invalidate_graph();
 }
 
-// Times the variants of k3_solve and k3_zbwd on this solver's own buffers (HIP events,
+// Times the variants of k3_tau_solve and k3_zbwd on this solver's own buffers (HIP events,
 // medians of 7 launches alternating with the default's) at creation.  A variant replaces the
 // default only when it is at least 3 % faster, so timing noise does not flip the choice.  The
 // choices are cached per (nx, ny, nz, dtype, solve form, |k_h|^2 keys) for the life of the process;
@@ -367,55 +316,26 @@ double Channel3Solver::implicit_c(bool first) const {
     return (1.0 + w) * d_.dt / (1.0 + 2.0 * w);
 }
 
+TauSys Channel3Solver::tau_sys() const {
+    return TauSys{d_.nz, tau_shape(d_.nz, true), nkeys_, factored_c_, 2.0 / d_.Lz, d_.kappa, d_.nu,
+                  kh_.as<const double>(), 0.0, tab_tau_.as<double>()};
+}
+
 void Channel3Solver::factor(double c) {
     if (c == factored_c_) return;
-    hipStream_t s = ctx_->stream;
-    const int N = d_.nz;
-    const size_t sb = (size_t)nb_max_ * nb_max_, su = (size_t)nu_max_ * nu_max_;
-    const unsigned nsys = (unsigned)(2 * nkeys_);
-    // assemble and LU-factor in scratch buffers, then keep only the explicit inverses
-    DevBuf Lb(ctx_, nsys * sb * sizeof(double)), Lp(ctx_, nsys * sb * sizeof(double)),
-        Lu(ctx_, nsys * su * sizeof(double));
-    DevBuf pb(ctx_, nsys * (size_t)nb_max_ * sizeof(int)), pp(ctx_, nsys * (size_t)nb_max_ * sizeof(int)),
-        pu(ctx_, nsys * (size_t)nu_max_ * sizeof(int));
-    Ch3Sys sys{N, nkeys_, sb, su, kh_.as<const double>(), 2.0 / d_.Lz, d_.kappa, d_.nu, c, d_.Lx * d_.Ly, d_.Lz};
-    hipLaunchKernelGGL(k3_assemble, dim3(nsys, 3), dim3(256), 0, s, sys, Lb.as<double>(), Lu.as<double>(),
-                       Lp.as<double>());
-    TG_HIP(hipGetLastError());
-    int* info = info_.as<int>();
-    constexpr int NT = 256;
-    hipLaunchKernelGGL((k_lu_factor_blocked<NT>), dim3(nsys), dim3(NT), (size_t)nb_max_ * 8, s, Lb.as<double>(),
-                       pb.as<int>(), info, N, 0, sb, (size_t)nb_max_);
-    hipLaunchKernelGGL((k_lu_factor_blocked<NT>), dim3(nsys), dim3(NT), (size_t)nb_max_ * 8, s, Lp.as<double>(),
-                       pp.as<int>(), info + nsys, N, 0, sb, (size_t)nb_max_);
-    hipLaunchKernelGGL((k_lu_factor_blocked<NT>), dim3(nsys), dim3(NT), (size_t)nu_max_ * 8, s, Lu.as<double>(),
-                       pu.as<int>(), info + 2 * nsys, N, 1, su, (size_t)nu_max_);
-    TG_HIP(hipGetLastError());
-    auto invert = [&](auto ot) {
-        using OT = decltype(ot);
-        const bool pack = d_.dtype == kF32;
-        lu_invert<NT, OT>(s, Lb.as<const double>(), pb.as<const int>(), Ib_.as<OT>(), N, 0, nsys, sb, nb_max_, nb_max_,
-                          pack, Iblo_.as<signed char>());
-        lu_invert<NT, OT>(s, Lp.as<const double>(), pp.as<const int>(), Ip_.as<OT>(), N, 0, nsys, sb, nb_max_, nb_max_,
-                          pack, Iplo_.as<signed char>());
-        lu_invert<NT, OT>(s, Lu.as<const double>(), pu.as<const int>(), Iu_.as<OT>(), N, 1, nsys, su, nu_max_, nu_max_,
-                          pack, Iulo_.as<signed char>());
-    };
-    if (d_.dtype == kF32) invert(float{});
-    else invert(double{});
-    TG_HIP(hipGetLastError());
-    std::vector<int> h((size_t)3 * nsys);
-    TG_HIP(hipMemcpyAsync(h.data(), info, h.size() * sizeof(int), hipMemcpyDeviceToHost, s));
-    TG_HIP(hipStreamSynchronize(s));
+    // a vanishing diffusivity leaves the D T_{N-1} lift of its equation without a coefficient
     std::string bad;
-    const char* names[3] = {" b-system", " perp-system", " u-p-system"};
-    for (int kind = 0; kind < 3; ++kind)
-        for (unsigned w = 0; w < nsys && bad.size() < 200; ++w)
-            if (h[kind * nsys + w])
-                bad += std::string(names[kind]) + "(|k_h| key " + std::to_string(w / 2) + ", parity " +
-                       std::to_string(w % 2) + ")";
+    const std::string par = ", parity " + std::to_string((d_.nz & 1) ? 1 : 0) + ")";  // parity of N - 2
+    for (int k = 0; k < nkeys_ && bad.size() < 200; ++k) {
+        const std::string key = "(|k_h| key " + std::to_string(k) + par;
+        if (d_.kappa == 0.0) bad += " b-system" + key;
+        if (d_.nu == 0.0) bad += " perp-system" + key + " u-p-system" + key;
+    }
     TG_REQUIRE(bad.empty(), kErrSingular, "3-D channel solver: singular per-mode system:" + bad);
     factored_c_ = c;
+    hipLaunchKernelGGL(k_tau_setup, dim3(nkeys_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream,
+                       tau_sys());
+    TG_HIP(hipGetLastError());
     invalidate_graph();
 }
 
@@ -530,38 +450,41 @@ void Channel3Solver::sbdf_t(bool first) {
 template <typename T>
 void Channel3Solver::solve_t() {
     using V = cplx<T>;
-    const int N = d_.nz;
-    Ch3SolveArgs sa{Ib_.ptr, Ip_.ptr, Iu_.ptr, Iblo_.as<const signed char>(), Iplo_.as<const signed char>(),
-                    Iulo_.as<const signed char>(),
-                    chunks_.as<const int4>(), modes_.as<const int>(), rot_.as<const double>(), N,
-                    sb_, su_, factored_c_, bcv_.as<const double2>(),
-                    d_.refine_sweeps, kh_.as<const double>(), d_.kappa, d_.nu, 2.0 / d_.Lz, d_.Lx * d_.Ly, d_.Lz};
-    // four wavefronts (at most 3 b/perp and 7 u-p tiles each for nz <= 256), or eight
-    const size_t lds = ch3_solve_lds_doubles(N, d_.refine_sweeps > 0) * sizeof(double);
+    TauArgs<T> a{};
+    a.t = tau_sys();
+    a.nmodes = nmodes_;
+    a.bcv = bcv_.as<const double2>();
+    a.modes = modes_.as<const int2>();
+    a.rot = rot_.as<const double>();
+    a.psi = tau_uses_psi(d_.nz, factored_c_, 2.0 / d_.Lz, d_.kappa, d_.nu, kh_max_);
+    a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
+    a.R2 = R_[1].as<const V>();
+    a.R3x = R_[2].as<const V>();
+    a.R3y = R_[3].as<const V>();
+    a.R3z = R_[4].as<const V>();
+    a.P = P_.as<V>();
+    a.B = B_.as<V>();
+    a.UX = UX_.as<V>();
+    a.UY = UY_.as<V>();
+    a.UZ = UZ_.as<V>();
+    a.taus = TAU_.as<V>();
+    const TauShape h = a.t.shape;
+    auto launch = [&](auto GC, auto EC) {
+        constexpr int G = decltype(GC)::value, E = decltype(EC)::value;
+        const unsigned np = tune_.solve == 1 ? 2 : 1, per = np * 64 / G;  // pairs of waves per workgroup
+        const dim3 grid((nmodes_ + per - 1) / per), block(128 * np);
+        const size_t lds = np * (tau_pair_bytes<G, E>() + tau_park_bytes<G, E>());
+        auto go = [&](auto psi, auto hasd) {
+            hipLaunchKernelGGL((k3_tau_solve<T, G, E, decltype(psi)::value, decltype(hasd)::value>), grid, block, lds,
+                               ctx_->stream, a);
+        };
+        tau_flags(a.psi, a.R1 != nullptr, go);
+    };
     timed(6, [&] {
-        auto launch = [&](auto kern, int nt) {
-            hipLaunchKernelGGL(kern, dim3(nchunks_), dim3(nt), lds, ctx_->stream, sa, R_[0].as<const V>(),
-                               R_[1].as<const V>(), R_[2].as<const V>(), R_[3].as<const V>(), R_[4].as<const V>(),
-                               P_.as<V>(), B_.as<V>(), UX_.as<V>(), UY_.as<V>(), UZ_.as<V>(), TAU_.as<V>());
-        };
-        auto by_size = [&](auto refine, auto split) {
-            constexpr bool R = decltype(refine)::value, S = decltype(split)::value;
-            const bool small = ch3_solve_small(nb_max_, nu_max_);
-            if (tune_.solve == 1) launch(k3_solve<T, 512, R, S, true>, 512);  // 8 waves: small tiles per wave
-            else if (small) launch(k3_solve<T, 256, R, S, true>, 256);
-            else launch(k3_solve<T, 256, R, S, false>, 256);
-        };
-        using yes = std::true_type;
-        using no = std::false_type;
-        if constexpr (sizeof(T) == 4) {
-            if (d_.split_inverse) {
-                if (d_.refine_sweeps > 0) by_size(yes{}, yes{});
-                else by_size(no{}, yes{});
-                return;
-            }
-        }
-        if (d_.refine_sweeps > 0) by_size(yes{}, no{});
-        else by_size(no{}, no{});
+        if (h.G == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 4>{});
+        else if (h.E == 4) launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 4>{});
+        else if (h.E == 2) launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 2>{});
+        else launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
     });
     TG_HIP(hipGetLastError());
 }
@@ -766,16 +689,8 @@ void Channel3Solver::kernel_bytes(double* out) const {
     out[3] = (4 * pad + 4 * nc) * vb;                           // read 4 padded planes, write 4
     out[4] = (8 * nc) * vb + N * N * rb;                        // read 4 planes, write 4 rows
     out[5] = (4 * 4 + 4 + 5) * nc * vb;                         // state (x2 on the kx lines), F, histories, rhs
-    double fac = 0;  // every chunk of up to 8 modes reads its key's three inverses once
-    const double eb = rb + (d_.split_inverse ? 1.0 : 0.0);  // bytes per inverse entry
-    for (int k = 0; k < nkeys_; ++k) {
-        const double chunks = (key_count_[k] + kCh3ChunkModes - 1) / kCh3ChunkModes;
-        for (int g = 0; g < 2; ++g) {
-            const double nb = chb_size(d_.nz, g ^ 1), np = chb_size(d_.nz, g), nu = chu_size(d_.nz, g, k);
-            fac += chunks * (nb * nb + np * np + nu * nu) * eb;
-        }
-    }
-    out[6] = fac + 10 * nc * vb;
+    // solve: rhs rows and the per-key tables in, five fields out
+    out[6] = (multistep() ? 9 : 10) * nc * vb + (double)nkeys_ * tau_table_stride(tau_shape(d_.nz, true)) * sizeof(double);
     out[7] = 10 * nc * vb;  // L x: read p, b, u (and partners on two lines), write five rows
 }
 
@@ -786,25 +701,19 @@ double Channel3Solver::nusselt() {
 }
 
 size_t footprint(const Channel3Desc& d) {
-    // every buffer the constructor allocates, in 2 MiB pages, plus the set-up scratch
+    // every buffer the constructor allocates, in 2 MiB pages
     const size_t nxh = d.nx / 2 + 1, nmodes = nxh * d.ny, N = d.nz, vb = 2 * dtype_size((DType)d.dtype);
     const size_t fb = nmodes * N * vb, prow = N * (size_t)padded_len(d.ny) * nxh * vb, ib = dtype_size((DType)d.dtype);
     const bool ms = d.stepper == kSBDF2 || d.stepper == kSBDF1;
     const size_t S = ms ? 0 : (size_t)make_tableau(d.stepper).stages;
     const size_t nfields = 5 + 12 + 5 + (ms ? 0 : 4 + 9 * S);  // state, history, rhs rows, RK stage rows
-    const size_t nb = chb_size(d.nz, 0), nu = chu_size(d.nz, 0, 0);
     // distinct |k_h|^2 keys: at most one per mode (about nmodes / 5.6 at 256 x 256 when Lx == Ly)
-    const size_t keys = d.Lx == d.Ly ? nmodes / 3 + 64 : nmodes, nsys = 2 * keys;
+    const size_t keys = d.Lx == d.Ly ? nmodes / 3 + 64 : nmodes;
     size_t b = nfields * alloc_granule(fb) + alloc_granule(kCh3Planes * fb) + alloc_granule(kCh3Planes * prow) +
                alloc_granule(4 * prow);                                                           // G, Q, H
     b += alloc_granule(nmodes * kCh3TauStride * vb) + 3 * alloc_granule(N * N * ib);           // taus, tables
-    const bool pack = d.dtype == kF32;
-    const size_t sb = inverse_stride((int)nb, pack), su = inverse_stride((int)nu, pack);
-    b += 2 * alloc_granule(nsys * sb * ib) + alloc_granule(nsys * su * ib);                     // inverses
-    if (d.split_inverse) b += 2 * alloc_granule(nsys * sb) + alloc_granule(nsys * su);  // remainders
-    b += 6 * alloc_granule(nmodes * 16);                                                      // keys, rotations, walls
-    b += 2 * alloc_granule(nsys * nb * nb * 8) + alloc_granule(nsys * nu * nu * 8) +
-         alloc_granule(nsys * (2 * nb + nu) * 4);                                             // FP64 LU scratch
+    b += alloc_granule(tau_table_doubles(tau_shape(d.nz, true), keys) * sizeof(double));  // tau-solve tables
+    b += 8 * alloc_granule(nmodes * 32);                                 // keys, rotations, modes, walls
     return b;
 }
 

@@ -1,10 +1,9 @@
 // channel3d_solver.hpp -- 3-D Rayleigh-Benard convection on RealFourier(x) x
 // RealFourier(y) x ChebyshevT(z) with the Chebyshev-tau method, per-mode
 // multistep (SBDF1/SBDF2) or IMEX Runge-Kutta stepping on the GPU.  Per (kx, ky) mode
-// the implicit system is solved through three FP64 systems that depend on |k_h| only
-// (buoyancy, the velocity normal to k_h, and the u-p system along k_h), each split
-// by parity; modes with equal |k_h|^2 share one explicit inverse per system, applied
-// to up to 8 modes at once on the FP64 matrix cores.
+// the implicit system splits into tridiagonal lines per field and parity (buoyancy, the
+// velocity normal to k_h and along it, pressure), solved directly in FP64 (tau_solve.hpp);
+// modes with equal |k_h|^2 share one small table.
 #pragma once
 #include <vector>
 
@@ -13,6 +12,7 @@
 
 namespace tarang {
 
+struct TauSys;
 struct Channel3Desc {
     int nx, ny, nz;
     double Lx, Ly, Lz;
@@ -21,9 +21,9 @@ struct Channel3Desc {
     int dtype;               // kF32 / kF64 (state, RHS, stage arithmetic; solves are FP64)
     int stepper;             // kSBDF2 / kSBDF1 (per-mode multistep) or kRK222 / kRK443 (IMEX RK)
     double b_bottom, b_top;  // Dirichlet values of b at z = 0 and z = Lz
-    int refine_sweeps = 0;   // FP64-residual refinement sweeps per implicit solve (0..2)
-    // FP32 state only: each inverse entry stored as an FP32 value plus an 8-bit
-    // remainder (2^-32 relative instead of 2^-24; 5 bytes per entry instead of 4)
+    // accepted (0..2, and 0 / 1 with an FP32 state) for callers of the stored-inverse solves; the
+    // direct FP64 solves hold no rounded inverse that a sweep or a remainder would correct
+    int refine_sweeps = 0;
     int split_inverse = 0;
 };
 
@@ -31,7 +31,7 @@ enum Channel3Var : int { kC3P = 0, kC3B = 1, kC3UX = 2, kC3UY = 3, kC3UZ = 4 };
 
 // kernel variants picked by the autotuner at creation; every variant gives the same bits
 struct Chan3Tuning {
-    int solve = 0;  // k3_solve workgroup: 0 four wavefronts, 1 eight
+    int solve = 0;  // k3_tau_solve workgroup: 0 one wave, 1 four
     int zbwd = 0;   // k3_zbwd mode tile: 0 the type's default (32 FP32 / 16 FP64), 1 16 modes (FP32 only)
 };
 
@@ -81,6 +81,7 @@ class Channel3Solver {
     template <typename T> void transpose_t(const void* in, void* out, int rows, int cols);
     double implicit_c(bool first) const;
     bool first_step() const { return multistep() && (iter_ == 0 || d_.stepper == kSBDF1); }
+    TauSys tau_sys() const;
     void factor(double c);
     void autotune();
     void launch_step_body();
@@ -94,7 +95,7 @@ class Channel3Solver {
 
     Context* ctx_;
     Channel3Desc d_;
-    int nxh_, nmodes_, mx_, my_, nb_max_, nu_max_, nkeys_ = 0;
+    int nxh_, nmodes_, mx_, my_, nkeys_ = 0;
     double factored_c_ = -1, dt_prev_ = 0, t_ = 0;
     long iter_ = 0;
     DevBuf P_, B_, UX_, UY_, UZ_, TAU_;
@@ -103,15 +104,11 @@ class Channel3Solver {
     DevBuf X0_[4], Frk_[4][4], LX_[4][5];  // IMEX RK stage storage
     DevBuf G_, Q_, H_;
     DevBuf BT_, BDT_, FT_;
-    DevBuf kh_, rot_, modes_, chunks_;
+    DevBuf kh_, rot_, modes_;
     DevBuf bcv_, bch_;  // per-mode wall values of b [2 m + w], and the x-transform scratch
-    // explicit inverses per (key, parity) of the b, perp and u-p systems: FP64 column-major,
-    // or FP32 packed (pk_index) with the 8-bit remainders in the *lo_ buffers when split
-    DevBuf Ib_, Ip_, Iu_, Iblo_, Iplo_, Iulo_, info_;
-    size_t sb_ = 0, su_ = 0;  // per-system strides of the inverses
+    DevBuf tab_tau_;  // per-key tables of the direct tau solves (tau_table_stride(nz) doubles each)
     Chan3Tuning tune_;
-    int nchunks_ = 0;
-    std::vector<int> key_count_;  // modes per key (host copy, for the byte model)
+    double kh_max_ = 0;
     bool graph_on_ = true;
     hipGraphExec_t graph_ = nullptr;
     double graph_dt_ = 0, graph_dtp_ = 0;

@@ -52,8 +52,6 @@ ChannelSolver::ChannelSolver(Context* ctx, const ChannelDesc& d) : ctx_(ctx), d_
     validate(d);
     nxh_ = d.nx / 2 + 1;
     mx_ = padded_len(d.nx);
-    nb_max_ = chb_size(d.nz, 0);
-    nu_max_ = chu_size(d.nz, 0, 0);
     tab_ = make_tableau(d.stepper);
     gamma_ = multistep() ? 0.0 : tab_.AI[1][1];
     dt_prev_ = d.dt;
@@ -102,17 +100,7 @@ ChannelSolver::ChannelSolver(Context* ctx, const ChannelDesc& d) : ctx_(ctx), d_
     upload(BT_, BT);
     upload(BDT_, BDT);
     upload(FT_, FT);
-    // two parity systems per mode and block
-    const size_t ib = dtype_size((DType)d.dtype);  // inverses in the state precision
-    Ib_ = DevBuf(ctx_, (size_t)2 * nxh_ * nb_max_ * nb_max_ * ib);
-    Iu_ = DevBuf(ctx_, (size_t)2 * nxh_ * nu_max_ * nu_max_ * ib);
-    if (d.split_inverse) {  // remainders in column quads; the slots past the last column stay zero
-        Iblo_ = DevBuf(ctx_, (size_t)2 * nxh_ * lo_quad_stride(nb_max_));
-        Iulo_ = DevBuf(ctx_, (size_t)2 * nxh_ * lo_quad_stride(nu_max_));
-        TG_HIP(hipMemsetAsync(Iblo_.ptr, 0, Iblo_.bytes, ctx_->stream));
-        TG_HIP(hipMemsetAsync(Iulo_.ptr, 0, Iulo_.bytes, ctx_->stream));
-    }
-    info_ = DevBuf(ctx_, (size_t)4 * nxh_ * sizeof(int));
+    tab_tau_ = DevBuf(ctx_, tau_table_doubles(tau_shape(d.nz, false), nxh_) * sizeof(double));
     {
         const auto bcv = constant_wall_values((size_t)nxh_, (double)d.nx, d.b_bottom, d.b_top);
         bcv_ = DevBuf(ctx_, bcv.size() * sizeof(double2));
@@ -218,45 +206,20 @@ void ChannelSolver::set_dt(double dt) {
 // ---- implicit systems ----
 void ChannelSolver::factor(double c) {
     if (c == factored_c_) return;
-    const int N = d_.nz;
-    hipStream_t s = ctx_->stream;
-    const size_t sb = (size_t)nb_max_ * nb_max_, su = (size_t)nu_max_ * nu_max_;
-    const unsigned nsys = (unsigned)(2 * nxh_);
-    // assemble and LU-factor in FP64 scratch buffers, then keep only the explicit inverses
-    DevBuf Lb(ctx_, nsys * sb * sizeof(double)), Lu(ctx_, nsys * su * sizeof(double));
-    DevBuf pb(ctx_, nsys * (size_t)nb_max_ * sizeof(int)), pu(ctx_, nsys * (size_t)nu_max_ * sizeof(int));
-    ChSys sys{N, nxh_, sb, su, 2.0 * M_PI / d_.Lx, 2.0 / d_.Lz, d_.kappa, d_.nu, c, d_.Lx, d_.Lz};
-    hipLaunchKernelGGL(k_ch_assemble, dim3(nsys, 2), dim3(256), 0, s, sys, Lb.as<double>(), Lu.as<double>());
-    TG_HIP(hipGetLastError());
-    int* info = info_.as<int>();
-    constexpr int NT = 256;
-    hipLaunchKernelGGL((k_lu_factor_blocked<NT>), dim3(nsys), dim3(NT), (size_t)nb_max_ * 8, s, Lb.as<double>(),
-                       pb.as<int>(), info, N, 0, sb, (size_t)nb_max_);
-    hipLaunchKernelGGL((k_lu_factor_blocked<NT>), dim3(nsys), dim3(NT), (size_t)nu_max_ * 8, s, Lu.as<double>(),
-                       pu.as<int>(), info + nsys, N, 1, su, (size_t)nu_max_);
-    TG_HIP(hipGetLastError());
-    auto invert = [&](auto ot) {
-        using OT = decltype(ot);
-        lu_invert<NT, OT>(s, Lb.as<const double>(), pb.as<const int>(), Ib_.as<OT>(), N, 0, nsys, sb, nb_max_, nb_max_,
-                          false, Iblo_.as<signed char>());
-        lu_invert<NT, OT>(s, Lu.as<const double>(), pu.as<const int>(), Iu_.as<OT>(), N, 1, nsys, su, nu_max_, nu_max_,
-                          false, Iulo_.as<signed char>());
-    };
-    if (d_.dtype == kF32) invert(float{});
-    else invert(double{});
-    TG_HIP(hipGetLastError());
-    std::vector<int> h((size_t)2 * nsys);
-    TG_HIP(hipMemcpyAsync(h.data(), info, h.size() * sizeof(int), hipMemcpyDeviceToHost, s));
-    TG_HIP(hipStreamSynchronize(s));
+    // a vanishing diffusivity leaves the D T_{N-1} lift of its equation without a coefficient
     std::string bad;
-    for (unsigned w = 0; w < nsys; ++w) {
-        const std::string mode = "(kx mode " + std::to_string(w / 2) + ", parity " + std::to_string(w % 2) + ")";
-        if (h[w]) bad += " b-system" + mode;
-        if (h[nsys + w]) bad += " u-p-system" + mode;
-        if (bad.size() > 200) break;
+    const int gb = (d_.nz & 1) ? 1 : 0;  // parity of N - 2
+    const std::string par = ", parity " + std::to_string(gb) + ")";
+    for (int m = 0; m < nxh_ && bad.size() < 200; ++m) {
+        const std::string mode = "(kx mode " + std::to_string(m) + par;
+        if (d_.kappa == 0.0) bad += " b-system" + mode;
+        if (d_.nu == 0.0) bad += " u-p-system" + mode;
     }
     TG_REQUIRE(bad.empty(), kErrSingular, "channel solver: singular per-mode system:" + bad);
     factored_c_ = c;
+    hipLaunchKernelGGL(k_tau_setup, dim3(nxh_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream,
+                       solve_args<double>().t);
+    TG_HIP(hipGetLastError());
     invalidate_graph();
 }
 
@@ -360,42 +323,51 @@ void ChannelSolver::stage_rhs_t(int st, bool final_update) {
     TG_HIP(hipGetLastError());
 }
 
-ChSolveArgs ChannelSolver::solve_args() const {
-    return ChSolveArgs{Ib_.ptr, Iu_.ptr, Iblo_.as<const signed char>(), Iulo_.as<const signed char>(),
-                       lo_quad_stride(nb_max_), lo_quad_stride(nu_max_), d_.nz, nxh_, (size_t)nb_max_ * nb_max_,
-                       (size_t)nu_max_ * nu_max_, nu_max_, factored_c_, bcv_.as<const double2>(), d_.refine_sweeps,
-                       2.0 * M_PI / d_.Lx, d_.kappa, d_.nu, 2.0 / d_.Lz, d_.Lx, d_.Lz};
+template <typename T>
+TauArgs<T> ChannelSolver::solve_args() const {
+    using V = cplx<T>;
+    TauArgs<T> a{};
+    const double k0x = 2.0 * M_PI / d_.Lx, sz = 2.0 / d_.Lz;
+    a.t = TauSys{d_.nz, tau_shape(d_.nz, false), nxh_, factored_c_, sz, d_.kappa, d_.nu, nullptr, k0x,
+                 tab_tau_.as<double>()};
+    a.nmodes = nxh_;
+    a.bcv = bcv_.as<const double2>();
+    a.psi = tau_uses_psi(d_.nz, factored_c_, sz, d_.kappa, d_.nu, k0x * (nxh_ - 1));
+    a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
+    a.R2 = R_[1].as<const V>();
+    a.R3x = R_[2].as<const V>();
+    a.R3z = R_[3].as<const V>();
+    a.P = P_.as<V>();
+    a.B = B_.as<V>();
+    a.UX = UX_.as<V>();
+    a.UZ = UZ_.as<V>();
+    a.taus = TAU_.as<V>();
+    return a;
+}
+
+int ChannelSolver::solve_wgs() const {
+    const int per = 64 / tau_shape(d_.nz, false).G;
+    return (nxh_ + per - 1) / per;
 }
 
 template <typename T>
 void ChannelSolver::solve_t() {
-    using V = cplx<T>;
-    const ChSolveArgs sa = solve_args();
-    constexpr int NT = 256;
-    const size_t lds = ch_solve_lds_doubles(nu_max_, d_.refine_sweeps > 0) * sizeof(double);
+    const TauArgs<T> sa = solve_args<T>();
+    const TauShape h = sa.t.shape;
+    const unsigned nwg = (unsigned)solve_wgs();
+    auto launch = [&](auto GC, auto EC) {
+        constexpr int G = decltype(GC)::value, E = decltype(EC)::value;
+        auto go = [&](auto psi, auto hasd) {
+            hipLaunchKernelGGL((k_ch_tau_solve<T, G, E, decltype(psi)::value, decltype(hasd)::value>), dim3(nwg),
+                               dim3(128), 0, ctx_->stream, sa);
+        };
+        tau_flags(sa.psi, sa.R1 != nullptr, go);
+    };
     timed(4, [&] {
-        auto launch = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(2 * nxh_), dim3(NT), lds, ctx_->stream, sa, R_[0].as<const V>(),
-                               R_[1].as<const V>(), R_[2].as<const V>(), R_[3].as<const V>(), P_.as<V>(), B_.as<V>(),
-                               UX_.as<V>(), UZ_.as<V>(), TAU_.as<V>());
-        };
-        // rows per thread: 2 covers every system up to 512 unknowns (nz <= 340)
-        auto by_size = [&](auto refine, auto split) {
-            constexpr bool R = decltype(refine)::value, S = decltype(split)::value;
-            if (nu_max_ <= 2 * NT) launch(k_ch_solve<T, NT, R, S, 2>);
-            else launch(k_ch_solve<T, NT, R, S, 4>);
-        };
-        using yes = std::true_type;
-        using no = std::false_type;
-        if constexpr (sizeof(T) == 4) {
-            if (d_.split_inverse) {
-                if (d_.refine_sweeps > 0) by_size(yes{}, yes{});
-                else by_size(no{}, yes{});
-                return;
-            }
-        }
-        if (d_.refine_sweeps > 0) by_size(yes{}, no{});
-        else by_size(no{}, no{});
+        if (h.G == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 1>{});
+        else if (h.E == 1) launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 1>{});
+        else if (h.E == 2) launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
+        else launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
     });
     TG_HIP(hipGetLastError());
 }
@@ -599,14 +571,8 @@ void ChannelSolver::kernel_bytes(double* out) const {
     out[1] = (8 * nc + 3 * nc) * vb;                    // read 8 planes, write 3
     out[2] = (3 * nc + 3 * nc) * vb + N * N * rb;       // read 3 planes, write 3 F
     out[3] = (4 * nc + 4 * nc) * vb;                    // read p, b, ux, uz; write 4 rows
-    // solve: read the four parity inverses per mode (state precision) and 4 rhs rows, write 4 fields
-    double fac = 0;
-    for (int m = 0; m < nxh_; ++m)
-        for (int g = 0; g < 2; ++g) {
-            const double nb = chb_size(d_.nz, g), nu = chu_size(d_.nz, g, m);
-            fac += (nb * nb + nu * nu) * (rb + (d_.split_inverse ? 1.0 : 0.0));
-        }
-    out[4] = fac + 8 * nc * vb;
+    // solve: read the rhs rows and the per-mode table, write 4 fields
+    out[4] = (multistep() ? 7 : 8) * nc * vb + (double)nxh_ * tau_table_stride(tau_shape(d_.nz, false)) * sizeof(double);
     out[5] = 0;
 }
 
@@ -617,21 +583,16 @@ double ChannelSolver::nusselt() {
 }
 
 size_t footprint(const ChannelDesc& d) {
-    // every buffer the constructor allocates, in 2 MiB pages, plus the set-up scratch
+    // every buffer the constructor allocates, in 2 MiB pages
     const size_t nxh = d.nx / 2 + 1, N = d.nz, vb = 2 * dtype_size((DType)d.dtype), fb = nxh * N * vb;
     const bool ms = d.stepper == kSBDF2 || d.stepper == kSBDF1;
     const size_t S = ms ? 0 : (size_t)make_tableau(d.stepper).stages;
     const size_t nfields = 4 + 3 + 4 + (ms ? 9 : 7 * S);  // state, X0, rhs rows, history or stage rows
-    const size_t nb = chb_size(d.nz, 0), nu = chu_size(d.nz, 0, 0), ib = dtype_size((DType)d.dtype);
-    const size_t nsys = 2 * nxh;
+    const size_t ib = dtype_size((DType)d.dtype);
     size_t b = nfields * alloc_granule(fb) + alloc_granule(8 * fb) + alloc_granule(3 * fb);  // G, H
     b += alloc_granule(nxh * 8 * vb) + 3 * alloc_granule(N * N * ib);                       // taus, tables
-    b += alloc_granule(nsys * nb * nb * ib) + alloc_granule(nsys * nu * nu * ib);            // inverses
-    if (d.split_inverse)  // remainders
-        b += alloc_granule(nsys * lo_quad_stride((int)nb)) + alloc_granule(nsys * lo_quad_stride((int)nu));
-    b += 3 * alloc_granule(1);                                                               // info, walls
-    // FP64 LU scratch and pivots while the inverses are formed
-    b += alloc_granule(nsys * nb * nb * 8) + alloc_granule(nsys * nu * nu * 8) + alloc_granule(nsys * (nb + nu) * 4);
+    b += alloc_granule(tau_table_doubles(tau_shape(d.nz, false), nxh) * sizeof(double));                    // tau-solve tables
+    b += 2 * alloc_granule(2 * nxh * sizeof(double2));                                       // walls
     return b;
 }
 
@@ -655,61 +616,37 @@ ChannelGroup::ChannelGroup(const std::vector<ChannelSolver*>& members) : m_(memb
                    kErrInvalid, "channel group: members must share dtype, timestepper, refine_sweeps and split_inverse");
     }
     ctx_ = m_[0]->ctx_;
-    for (ChannelSolver* s : m_) total_wg_ += 2 * s->nxh_;
+    for (ChannelSolver* s : m_) total_wg_ += s->solve_wgs();
 }
 
 ChannelGroup::~ChannelGroup() { invalidate_graph(); }
 
 template <typename T>
 void ChannelGroup::fill_items() {
-    using V = cplx<T>;
-    std::vector<ChSolveItem<T>> it(m_.size());
+    std::vector<TauItem<T>> it(m_.size());
     int wg0 = 0;
     for (size_t i = 0; i < m_.size(); ++i) {
         ChannelSolver* s = m_[i];
-        it[i].s = s->solve_args();
-        for (int r = 0; r < 4; ++r) it[i].R[r] = s->R_[r].as<const V>();
-        it[i].out[0] = s->P_.as<V>();
-        it[i].out[1] = s->B_.as<V>();
-        it[i].out[2] = s->UX_.as<V>();
-        it[i].out[3] = s->UZ_.as<V>();
-        it[i].out[4] = s->TAU_.as<V>();
+        it[i].s = s->solve_args<T>();
         it[i].wg0 = wg0;
-        wg0 += 2 * s->nxh_;
+        wg0 += s->solve_wgs();
     }
-    hitems_.resize(it.size() * sizeof(ChSolveItem<T>));
+    int psi = 0;  // one kernel for the group: the psi-form variant when any member needs it
+    for (auto& i : it) psi |= i.s.psi;
+    for (auto& i : it) i.s.psi = psi;
+    hitems_.resize(it.size() * sizeof(TauItem<T>));
     std::memcpy(hitems_.data(), it.data(), hitems_.size());
 }
 
 template <typename T>
 void ChannelGroup::solve_group_t() {
-    constexpr int NT = 256;
-    const ChannelDesc& d = m_[0]->d_;
-    int nu_max = 0;
-    for (ChannelSolver* s : m_) nu_max = std::max(nu_max, s->nu_max_);
-    const size_t lds = ch_solve_lds_doubles(nu_max, d.refine_sweeps > 0) * sizeof(double);
-    const ChSolveItem<T>* items = items_.as<const ChSolveItem<T>>();
+    const TauItem<T>* items = items_.as<const TauItem<T>>();
     const int n = (int)m_.size();
-    auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(total_wg_), dim3(NT), lds, ctx_->stream, items, n); };
-    auto by_size = [&](auto refine, auto split) {  // as ChannelSolver::solve_t, for the largest member
-        constexpr bool R = decltype(refine)::value, S = decltype(split)::value;
-        if (nu_max <= 2 * NT) launch(k_ch_solve_group<T, NT, R, S, 2>);
-        else launch(k_ch_solve_group<T, NT, R, S, 4>);
-    };
-    using yes = std::true_type;
-    using no = std::false_type;
-    bool done = false;
-    if constexpr (sizeof(T) == 4) {
-        if (d.split_inverse) {
-            if (d.refine_sweeps > 0) by_size(yes{}, yes{});
-            else by_size(no{}, yes{});
-            done = true;
-        }
-    }
-    if (!done) {
-        if (d.refine_sweeps > 0) by_size(yes{}, no{});
-        else by_size(no{}, no{});
-    }
+    const TauArgs<T>& first = reinterpret_cast<const TauItem<T>*>(hitems_.data())->s;  // flags group-wide (fill_items)
+    tau_flags(first.psi, first.R1 != nullptr, [&](auto psi, auto hasd) {
+        hipLaunchKernelGGL((k_ch_tau_solve_group<T, decltype(psi)::value, decltype(hasd)::value>), dim3(total_wg_),
+                           dim3(128), 0, ctx_->stream, items, n);
+    });
     TG_HIP(hipGetLastError());
 }
 

@@ -1,8 +1,8 @@
 // channel_solver.hpp -- 2-D Rayleigh-Benard convection on RealFourier(x) x
 // ChebyshevT(z) with the Chebyshev-tau method, stepped on the GPU with IMEX RK or
-// SBDF.  Per Fourier mode the implicit system splits into a buoyancy block and a
-// velocity-pressure block (each by parity); both are factored in FP64 once per
-// implicit coefficient and kept as explicit inverses in the state precision.
+// SBDF.  Per Fourier mode the implicit system splits into tridiagonal lines per field and
+// parity, solved directly in FP64 (tau_solve.hpp); a small table per mode is set up once
+// per implicit coefficient.
 #pragma once
 #include <vector>
 
@@ -19,15 +19,15 @@ struct ChannelDesc {
     int dtype;           // kF32 / kF64 (state and RHS; the implicit solves are FP64)
     int stepper;         // kRK222 / kRK443 / kSBDF2 / kSBDF1
     double b_bottom, b_top;  // Dirichlet values of b at z = 0 and z = Lz
-    int refine_sweeps = 0;   // FP64-residual refinement sweeps per implicit solve (0..2)
-    // FP32 state only: each inverse entry stored as an FP32 value plus an 8-bit
-    // remainder (2^-32 relative instead of 2^-24; 5 bytes per entry instead of 4)
+    // accepted (0..2, and 0 / 1 with an FP32 state) for callers of the stored-inverse solves; the
+    // direct FP64 solves hold no rounded inverse that a sweep or a remainder would correct
+    int refine_sweeps = 0;
     int split_inverse = 0;
 };
 
 enum ChannelVar : int { kChP = 0, kChB = 1, kChUX = 2, kChUZ = 3 };
 
-struct ChSolveArgs;
+template <typename T> struct TauArgs;
 class ChannelGroup;
 
 class ChannelSolver {
@@ -69,7 +69,8 @@ class ChannelSolver {
     int nsolves() const { return multistep() ? 1 : tab_.stages - 1; }
     void segment(int i);
     template <typename T> void segment_t(int i);
-    ChSolveArgs solve_args() const;
+    template <typename T> TauArgs<T> solve_args() const;
+    int solve_wgs() const;  // workgroups (waves) of the solve kernel
     void advance_clock();
     template <typename T> void rhs_t(const void* b, const void* ux, const void* uz, void* F0, void* F1, void* F2);
     template <typename T> void lx_t(int s);
@@ -95,7 +96,7 @@ class ChannelSolver {
 
     Context* ctx_;
     ChannelDesc d_;
-    int nxh_, mx_, nb_max_, nu_max_;
+    int nxh_, mx_;
     Tableau tab_;
     double gamma_ = 0, factored_c_ = -1;
     double t_ = 0;
@@ -105,13 +106,10 @@ class ChannelSolver {
     DevBuf F_[4][3], LX_[4][4], R_[4];
     DevBuf Fm1_[3], MXm1_[3];  // multistep history
     double dt_prev_ = 0;
-    double solve_c_ = 0;       // c of the factored systems used by the solve kernel
     DevBuf G_, H_;
     DevBuf BT_, BDT_, FT_;
     DevBuf bcv_, bch_;  // per-mode wall values of b [2 m + w], and the x-transform scratch
-    // explicit inverses per (mode, parity) of the b and u-p systems, state precision, with
-    // the 8-bit remainders of FP32 entries in the *lo_ buffers when split
-    DevBuf Ib_, Iu_, Iblo_, Iulo_, info_;
+    DevBuf tab_tau_;    // per-mode tables of the direct tau solves (tau_table_stride(nz) doubles each)
     bool graph_on_ = true;
     hipGraphExec_t graph_ = nullptr;
     double graph_dt_ = 0, graph_dtp_ = 0;
@@ -124,7 +122,7 @@ class ChannelSolver {
 // Several 2-D channel problems stepped together: one context, and the same dtype,
 // timestepper and solve form (refine_sweeps, split_inverse); any nx, nz, dt, Lx, Lz,
 // diffusivities and walls.  Each implicit stage runs the per-mode solves of every member
-// as one launch (k_ch_solve_group, workgroups over all members' modes); the group step
+// as one launch (k_ch_tau_solve_group, workgroups over all members' modes); the group step
 // is replayed as one hipGraph.  The members keep their own clocks and multistep history
 // and may still be stepped alone; they must outlive the group.
 class ChannelGroup {

@@ -6,10 +6,19 @@
 #include <string>
 #include <vector>
 
-#include "channel_kernels.hpp"  // MfmaOp, readlane_f64
+#include "common.hpp"
 #include "dense_ops.hpp"
+#include "mfma.hpp"
 
 namespace tarang {
+
+// value of v in lane `lane` (wave-uniform index), through scalar registers
+__device__ inline double readlane_f64(double v, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+
 
 // ===========================================================================
 // Dense operator along one axis, with the parity split of the Gauss-Lobatto grid.

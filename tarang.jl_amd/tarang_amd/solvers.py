@@ -67,9 +67,9 @@ class InitialValueSolver:
 
     Keyword arguments mirror the reference (`dt`, `matsolver`, `batched_modes`,
     ...); `use_graph` (default True) replays each step as one captured hipGraph.
-    Channel families only: `split_inverse` (default: on for an FP32 domain) stores the
-    per-mode inverses as FP32 values plus 8-bit remainders, and `refine_sweeps` (0-2)
-    adds FP64-residual refinement sweeps to every implicit solve.
+    Channel families only: `split_inverse` (default: on for an FP32 domain) and
+    `refine_sweeps` (0-2) are checked and passed on, but change nothing: the per-mode
+    solves are direct, in FP64 arithmetic, whatever the state's precision.
     """
 
     def __init__(self, problem: IVP, timestepper, dt: float, matsolver=None, use_graph: bool = True,
