@@ -325,15 +325,20 @@ void cheb_deriv(Context* c, const void* in, void* out, int ndim, const int* shap
 // Right-looking, blocked by panels of kLuNB columns.  Within a panel the columns
 // are factored one at a time in LAPACK's zgetf2 order: pivot = first row of
 // largest |Re| + |Im| (izamax), interchange, scale by the reciprocal pivot,
-// rank-1 update of the rest of the panel.  Then the panel's interchanges are
-// applied to the other columns, U12 = L11^{-1} A12 is formed 128 columns at a
-// time (one thread per column, the chunk kept in LDS) and the trailing matrix
-// takes the rank-kLuNB update A22 -= L21 U12 (threads along rows, so the
-// column-major matrix is read and written in contiguous runs).  An exactly zero
-// pivot column is recorded in info (first one, 1-based) and skipped, as LAPACK does.
+// rank-1 update of the rest of the panel.  The panel's rows live in registers, RPT of
+// them per thread (RPT = 0: in global memory, for matrices of more rows than that holds).
+// Then the panel's interchanges, composed into one permutation, are applied to the other
+// columns, U12 = L11^{-1} A12 is formed kLuCC columns at a time (one thread per column)
+// and the trailing matrix takes the rank-kLuNB update A22 -= L21 U12 on the matrix cores
+// (lanes along rows, so the column-major matrix is read and written in contiguous runs).
+// An exactly zero pivot column is recorded in info (first one, 1-based) and skipped, as
+// LAPACK does.
+// Bound: the chain of a column (two barriers, the reduction, a reciprocal: 5700 clocks with 512
+// threads), half of the 1280 us of 129 matrices of n = 263; the products take a third, at 0.4 of the
+// FP64 rate of their CU.  Before, panel and products from memory, thread by thread: 2965 us.
+// Whole calls: 1031 x 64 36 against 73 ms, 400 x 60 2.7 against 6.3 ms, 40 x 9 139 against 226 us.
 // ===========================================================================
 constexpr int kLuNB = 16;
-constexpr int kLuCC = 128;
 
 __device__ inline double cabs1(double2 z) { return fabs(z.x) + fabs(z.y); }
 __device__ inline double2 crecip(double2 z) {  // 1/z, Smith's scaling
@@ -345,55 +350,135 @@ __device__ inline double2 crecip(double2 z) {  // 1/z, Smith's scaling
     return double2{r / d, -1.0 / d};
 }
 
-template <int NT>
+// the larger value, of equal ones the smaller row
+__device__ inline void pivot_max(double& v, int& i, double ov, int oi) {
+    const bool take = ov > v || (ov == v && oi < i);
+    v = take ? ov : v;
+    i = take ? oi : i;
+}
+template <int CTRL>
+__device__ inline void pivot_max_dpp(double& v, int& i) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    pivot_max(v, i, __hiloint2double(hi, lo), __builtin_amdgcn_update_dpp(0, i, CTRL, 0xf, 0xf, true));
+}
+// over the wavefront, in every lane: rotations of the 16-lane rows, then the four rows
+__device__ inline void pivot_max_wave(double& v, int& i) {
+    pivot_max_dpp<0x128>(v, i);
+    pivot_max_dpp<0x124>(v, i);
+    pivot_max_dpp<0x122>(v, i);
+    pivot_max_dpp<0x121>(v, i);
+    double rv = readlane_f64(v, 0);
+    int ri = __builtin_amdgcn_readlane(i, 0);
+#pragma unroll
+    for (int r = 16; r < 64; r += 16) pivot_max(rv, ri, readlane_f64(v, r), __builtin_amdgcn_readlane(i, r));
+    v = rv;
+    i = ri;
+}
+
+template <int NT, int RPT>
 __global__ __launch_bounds__(NT) void k_zgetrf(double2* __restrict__ Aall, int n, int* __restrict__ ipiv_all,
                                                int* __restrict__ info_all) {
-    constexpr int NW = NT / 64;
-    __shared__ double red_v[NW];
-    __shared__ int red_i[NW];
-    __shared__ int piv_s[kLuNB];
-    __shared__ double2 l11[kLuNB * kLuNB];
-    __shared__ double2 u12[kLuNB * kLuCC];
+    constexpr int NW = NT / 64, NB = kLuNB, CC = NT < 256 ? NT : 256;
+    __shared__ double red_v[2][NW];
+    __shared__ int red_i[2][NW];
+    __shared__ int piv_s[NB];
+    __shared__ int mv_dst[2 * NB], mv_src[2 * NB];
+    __shared__ double2 rows_s[2][2][NB];  // [column parity][pivot row, row k]
+    __shared__ double2 l11[NB * NB];
+    __shared__ double2 u12[CC * (NB + 1)];  // [column][row], one column apart in bank
     const int m = blockIdx.x;
     double2* a = Aall + (size_t)m * n * n;
     int* ipiv = ipiv_all + (size_t)m * n;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     int bad = 0;
-    for (int k0 = 0; k0 < n; k0 += kLuNB) {
-        const int kb = min(kLuNB, n - k0);
-        for (int kk = 0; kk < kb; ++kk) {
-            const int k = k0 + kk;
+    for (int k0 = 0; k0 < n; k0 += NB) {
+        const int kb = min(NB, n - k0);
+        // ---- panel ----
+        double xr[RPT > 0 ? RPT : 1][NB], xi[RPT > 0 ? RPT : 1][NB];
+        auto get = [&](int j, int c) { return double2{xr[j][c], xi[j][c]}; };
+        auto set = [&](int j, int c, double2 v) { xr[j][c] = v.x, xi[j][c] = v.y; };
+        if constexpr (RPT > 0) {
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                const int i = k0 + t + j * NT;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) set(j, c, i < n && c < kb ? a[(size_t)(k0 + c) * n + i] : double2{0.0, 0.0});
+            }
+        }
+        // Column kk; with the panel in registers its values are x[.][S] and those of column kk + c - S are x[.][c],
+        // columns from kk + left on (cyclically: the finished ones) take no update
+        auto column = [&](auto SC, int kk, int left) __attribute__((always_inline)) {
+            constexpr int S = decltype(SC)::value;
+            const int k = k0 + kk, ph = kk & 1;
             double best = -1.0;
             int bi = n;
-            for (int i = k + t; i < n; i += NT) {
-                const double v = cabs1(a[(size_t)k * n + i]);
-                if (v > best) { best = v; bi = i; }
-            }
+            if constexpr (RPT > 0) {
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const double ov = __shfl_xor(best, off);
-                const int oi = __shfl_xor(bi, off);
-                if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+                for (int j = 0; j < RPT; ++j) {
+                    const int i = k0 + t + j * NT;
+                    const double v = cabs1(get(j, S));
+                    if (i >= k && i < n && v > best) { best = v; bi = i; }
+                }
+            } else {
+                for (int i = k + t; i < n; i += NT) {
+                    const double v = cabs1(a[(size_t)k * n + i]);
+                    if (v > best) { best = v; bi = i; }
+                }
             }
-            if (lane == 0) { red_v[w] = best; red_i[w] = bi; }
+            pivot_max_wave(best, bi);
+            if (lane == 0) { red_v[ph][w] = best; red_i[ph][w] = bi; }
             __syncthreads();
-            double pv = red_v[0];
-            int p = red_i[0];
+            double pv = red_v[ph][0];
+            int p = red_i[ph][0];
 #pragma unroll
-            for (int q = 1; q < NW; ++q)
-                if (red_v[q] > pv || (red_v[q] == pv && red_i[q] < p)) { pv = red_v[q]; p = red_i[q]; }
+            for (int q = 1; q < NW; ++q) pivot_max(pv, p, red_v[ph][q], red_i[ph][q]);
             if (p >= n) p = k;  // no comparable value (NaN column): keep the diagonal, as izamax does
             const bool zero = pv == 0.0;
-            if (t == 0) { ipiv[k] = p + 1; piv_s[kk] = p; }
-            if (zero) { if (!bad) bad = k + 1; }
-            else if (p != k && t < kb) {
-                double2* col = a + (size_t)(k0 + t) * n;
-                const double2 x = col[k];
-                col[k] = col[p];
-                col[p] = x;
+            if (t == 0) piv_s[kk] = p;  // to memory after the panel: a barrier waits for every store before it
+            if (zero) {
+                if (!bad) bad = k + 1;
+                return;  // every thread: the next column's reduction uses the other buffer
             }
-            __syncthreads();
-            if (!zero) {
+            if constexpr (RPT > 0) {
+#pragma unroll
+                for (int j = 0; j < RPT; ++j) {
+                    const int i = k0 + t + j * NT;
+                    if (i == p)
+#pragma unroll
+                        for (int c = 0; c < NB; ++c) rows_s[ph][0][c] = get(j, c);
+                    if (i == k)
+#pragma unroll
+                        for (int c = 0; c < NB; ++c) rows_s[ph][1][c] = get(j, c);
+                }
+                __syncthreads();
+                const double2 r = crecip(rows_s[ph][0][S]);
+#pragma unroll
+                for (int j = 0; j < RPT; ++j) {
+                    const int i = k0 + t + j * NT;
+                    if (p != k && (i == p || i == k)) {
+                        const double2* from = rows_s[ph][i == p ? 1 : 0];
+#pragma unroll
+                        for (int c = 0; c < NB; ++c) set(j, c, from[c]);
+                    }
+                    const bool below = i > k;
+                    const double2 l = cmul(get(j, S), r);
+                    if (below) set(j, S, l);
+#pragma unroll
+                    for (int c4 = 0; c4 < NB; c4 += 4)
+                        if (c4 < left && below)  // blocks of four columns: `left` is a multiple of four
+#pragma unroll
+                            for (int c = c4; c < c4 + 4; ++c)
+                                if (c > S) set(j, c, csub(get(j, c), cmul(l, rows_s[ph][0][c])));
+                }
+            } else {
+                if (p != k && t < kb) {
+                    double2* col = a + (size_t)(k0 + t) * n;
+                    const double2 y = col[k];
+                    col[k] = col[p];
+                    col[p] = y;
+                }
+                __syncthreads();
                 const double2 r = crecip(a[(size_t)k * n + k]);
                 for (int i = k + 1 + t; i < n; i += NT) {
                     const double2 l = cmul(a[(size_t)k * n + i], r);
@@ -403,52 +488,164 @@ __global__ __launch_bounds__(NT) void k_zgetrf(double2* __restrict__ Aall, int n
                         *e = csub(*e, cmul(l, a[(size_t)(k0 + c) * n + k]));
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
-        }
-        // the panel's interchanges on every other column, in order
-        for (int c = t; c < n; c += NT) {
-            if (c >= k0 && c < k0 + kb) continue;
-            double2* col = a + (size_t)c * n;
-            for (int q = 0; q < kb; ++q) {
-                const int p = piv_s[q];
-                if (p != k0 + q) {
-                    const double2 x = col[k0 + q];
-                    col[k0 + q] = col[p];
-                    col[p] = x;
+        };
+        if constexpr (RPT > 0) {
+            // four columns per turn of a loop, then the registers move on by four: a quarter of the code of
+            // sixteen written out, at the same time
+#pragma unroll 1
+            for (int kk = 0; kk < NB; kk += 4) {
+                const int left = NB - kk;
+                if (kk < kb) column(std::integral_constant<int, 0>{}, kk, left);
+                if (kk + 1 < kb) column(std::integral_constant<int, 1>{}, kk + 1, left);
+                if (kk + 2 < kb) column(std::integral_constant<int, 2>{}, kk + 2, left);
+                if (kk + 3 < kb) column(std::integral_constant<int, 3>{}, kk + 3, left);
+#pragma unroll
+                for (int j = 0; j < RPT; ++j) {
+                    double yr[4], yi[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) yr[c] = xr[j][c], yi[c] = xi[j][c];
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) {
+                        xr[j][c] = c + 4 < NB ? xr[j][(c + 4) % NB] : yr[c % 4];
+                        xi[j][c] = c + 4 < NB ? xi[j][(c + 4) % NB] : yi[c % 4];
+                    }
                 }
             }
-        }
-        for (int e = t; e < kLuNB * kLuNB; e += NT) {
-            const int c = e / kLuNB, r = e % kLuNB;
-            l11[e] = (c < kb && r < kb) ? a[(size_t)(k0 + c) * n + k0 + r] : double2{0.0, 0.0};
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                const int i = k0 + t + j * NT;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) {
+                    if (i < n && c < kb) a[(size_t)(k0 + c) * n + i] = get(j, c);
+                    if (j == 0 && t < NB) l11[c * NB + t] = get(0, c);
+                }
+            }
+        } else {
+            for (int kk = 0; kk < kb; ++kk) column(std::integral_constant<int, 0>{}, kk, 0);
+            for (int e = t; e < NB * NB; e += NT) {
+                const int c = e / NB, r = e % NB;
+                l11[e] = (c < kb && r < kb) ? a[(size_t)(k0 + c) * n + k0 + r] : double2{0.0, 0.0};
+            }
         }
         __syncthreads();
-        const int c1 = k0 + kb;
-        for (int cc0 = c1; cc0 < n; cc0 += kLuCC) {
-            const int cw = min(kLuCC, n - cc0);
-            if (t < cw) {  // U12 column: forward substitution with the unit lower L11, in LDS
-                double2* col = a + (size_t)(cc0 + t) * n + k0;
-                for (int q = 0; q < kLuNB; ++q) u12[q * kLuCC + t] = q < kb ? col[q] : double2{0.0, 0.0};
-                for (int r = 1; r < kb; ++r) {
-                    double2 acc = u12[r * kLuCC + t];
-                    for (int q = 0; q < r; ++q) acc = csub(acc, cmul(l11[q * kLuNB + r], u12[q * kLuCC + t]));
-                    u12[r * kLuCC + t] = acc;
-                    col[r] = acc;
+        // ---- the interchanges as one permutation: lane q < 16 holds row k0 + q, lane 16 + j the j-th row
+        // outside the block that takes part; row mv_dst takes the value of row mv_src ----
+        if (w == 0) {
+            const int mine = lane < kb ? piv_s[lane] : 0;
+            if (lane < kb) ipiv[k0 + lane] = mine + 1;
+            int row = lane < NB ? k0 + lane : -1, src = row, used = 0;
+            for (int q = 0; q < kb; ++q) {
+                const int p = __builtin_amdgcn_readlane(mine, q);
+                if (p == k0 + q) continue;
+                int b;
+                if (p < k0 + NB) b = p - k0;
+                else {
+                    const unsigned long long hit = __ballot(row == p);
+                    if (hit) b = __builtin_ctzll(hit);
+                    else {
+                        b = NB + used++;
+                        if (lane == b) row = src = p;
+                    }
                 }
+                const int sq = __builtin_amdgcn_readlane(src, q), sb = __builtin_amdgcn_readlane(src, b);
+                src = lane == q ? sb : (lane == b ? sq : src);
+            }
+            if (lane < 2 * NB) {
+                mv_dst[lane] = src == row ? -1 : row;
+                mv_src[lane] = src;
+            }
+        }
+        __syncthreads();
+        {
+            const int h = lane & 31, dst = mv_dst[h], src = dst >= 0 ? mv_src[h] : k0;
+            constexpr int PER = NT / 32, UN = 8;  // columns per round; rounds in flight
+            for (int cb = t >> 5; cb < n - kb; cb += PER * UN) {
+                double vx[UN], vy[UN];
+                auto col = [&](int u) {  // the panel's own columns are in place
+                    const int c = min(cb + u * PER, n - kb - 1);
+                    return a + (size_t)(c < k0 ? c : c + kb) * n;
+                };
+#pragma unroll
+                for (int u = 0; u < UN; ++u) {
+                    const double2 v = col(u)[src];
+                    vx[u] = v.x;
+                    vy[u] = v.y;
+                }
+#pragma unroll
+                for (int u = 0; u < UN; ++u)
+                    if (cb + u * PER < n - kb && dst >= 0) col(u)[dst] = double2{vx[u], vy[u]};
+            }
+        }
+        __syncthreads();
+        // ---- U12 and the trailing update; kb = NB here (a short panel is the last) ----
+        const int c1 = k0 + kb;
+        for (int cc0 = c1; cc0 < n; cc0 += CC) {
+            const int cw = min(CC, n - cc0);
+            if (t < CC) {  // U12 column: forward substitution with the unit lower L11
+                double2 u[NB];
+                double2* col = a + (size_t)(cc0 + t) * n + k0;
+#pragma unroll
+                for (int q = 0; q < NB; ++q) u[q] = t < cw ? col[q] : double2{0.0, 0.0};
+#pragma unroll
+                for (int q = 0; q < NB - 1; ++q) {
+                    int o = q * NB;  // L11 one column ahead: read all at once, its 120 entries would spill
+                    asm volatile("" : "+v"(o) : "v"(u[q > 0 ? q - 1 : 0].x));
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int r = q + 1; r < NB; ++r) u[r] = csub(u[r], cmul(l11[o + r], u[q]));
+                }
+#pragma unroll
+                for (int q = 0; q < NB; ++q) u12[t * (NB + 1) + q] = u[q];  // zero beyond cw
+                if (t < cw)
+#pragma unroll
+                    for (int q = 1; q < NB; ++q) col[q] = u[q];
             }
             __syncthreads();
-            for (int i = c1 + t; i < n; i += NT) {  // A22 -= L21 U12
-                double2 l[kLuNB];
+            // A22 -= L21 U12 in 16 x 16 tiles, D^T = U12^T L21^T: a lane's D column is a row of A22.  A wave
+            // takes a run of tiles, columns fastest, the next tile's A22 in flight during the products.
+            using Op = MfmaOp<double>;
+            const int nrt = (n - c1 + 15) >> 4, nct = (cw + 15) >> 4, ntile = nrt * nct;
+            const int per = (ntile + NW - 1) / NW, tb = w * per, te = min(ntile, tb + per);
+            const int i16 = lane & 15, q4 = lane >> 4;
+            double lr[4], li[4];
+            double2 cn[4];
+            auto fetch = [&](int tile) {
+                const int rt = tile / nct, ct = tile - rt * nct, i = c1 + 16 * rt + i16;
 #pragma unroll
-                for (int q = 0; q < kLuNB; ++q) l[q] = q < kb ? a[(size_t)(k0 + q) * n + i] : double2{0.0, 0.0};
-#pragma unroll 2
-                for (int c = 0; c < cw; ++c) {
-                    double2* e = a + (size_t)(cc0 + c) * n + i;
-                    double2 acc = *e;
+                for (int v = 0; v < 4; ++v) {
+                    const int c = 16 * ct + Op::row(v, q4);
+                    cn[v] = i < n && c < cw ? a[(size_t)(cc0 + c) * n + i] : double2{0.0, 0.0};
+                }
+            };
+            int have = -1;
+            if (tb < te) fetch(tb);
+            for (int tile = tb; tile < te; ++tile) {
+                const int rt = tile / nct, ct = tile - rt * nct, i = c1 + 16 * rt + i16;
+                if (rt != have) {
+                    have = rt;
 #pragma unroll
-                    for (int q = 0; q < kLuNB; ++q) acc = csub(acc, cmul(l[q], u12[q * kLuCC + c]));
-                    *e = acc;
+                    for (int s = 0; s < 4; ++s) {
+                        const double2 l = i < n ? a[(size_t)(k0 + 4 * s + q4) * n + i] : double2{0.0, 0.0};
+                        lr[s] = l.x;
+                        li[s] = l.y;
+                    }
+                }
+                Op::acc4 cr{cn[0].x, cn[1].x, cn[2].x, cn[3].x}, ci{cn[0].y, cn[1].y, cn[2].y, cn[3].y};
+                if (tile + 1 < te) fetch(tile + 1);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const double2 u = u12[(16 * ct + i16) * (NB + 1) + 4 * s + q4];
+                    cr = Op::mma(-u.x, lr[s], cr);
+                    ci = Op::mma(-u.x, li[s], ci);
+                    cr = Op::mma(u.y, li[s], cr);
+                    ci = Op::mma(-u.y, lr[s], ci);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int c = 16 * ct + Op::row(v, q4);
+                    if (i < n && c < cw) a[(size_t)(cc0 + c) * n + i] = double2{cr[v], ci[v]};
                 }
             }
             __syncthreads();
@@ -572,8 +769,19 @@ void zgetrf_batched(Context* c, void* A, int n, int nmodes, int* ipiv, int* info
     TG_REQUIRE(A != nullptr && ipiv != nullptr, kErrInvalid, "batched LU: NULL matrix or pivot buffer");
     c->activate();
     DevBuf info(c, sizeof(int) * (size_t)nmodes);
-    hipLaunchKernelGGL((k_zgetrf<512>), dim3((unsigned)nmodes), dim3(512), 0, c->stream, static_cast<double2*>(A), n,
-                       ipiv, info.as<int>());
+    auto launch = [&](auto nt, auto rpt) {
+        constexpr int NT = decltype(nt)::value, RPT = decltype(rpt)::value;
+        hipLaunchKernelGGL((k_zgetrf<NT, RPT>), dim3((unsigned)nmodes), dim3(NT), 0, c->stream,
+                           static_cast<double2*>(A), n, ipiv, info.as<int>());
+    };
+    // one panel row per thread while a workgroup has the threads, then two and three (the 16
+    // columns of a row are 64 registers of the 256 that 512 threads leave each); above, the
+    // panel stays in memory
+    if (n <= 128) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 1>{});
+    else if (n <= 256) launch(std::integral_constant<int, 256>{}, std::integral_constant<int, 1>{});
+    else if (n <= 512) launch(std::integral_constant<int, 512>{}, std::integral_constant<int, 1>{});
+    else if (n <= 1024) launch(std::integral_constant<int, 512>{}, std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 512>{}, std::integral_constant<int, 0>{});
     TG_HIP(hipGetLastError());
     std::vector<int> h((size_t)nmodes);
     TG_HIP(hipMemcpyAsync(h.data(), info.ptr, sizeof(int) * (size_t)nmodes, hipMemcpyDeviceToHost, c->stream));
