@@ -20,9 +20,14 @@
 
 namespace tarang {
 
-// operand planes of the 3-D right-hand side
-//   0 ux, 1 uy, 2 uz, then for f in (b, ux, uy, uz): 3+3f dx f, 4+3f dy f, 5+3f dz f
-constexpr int kCh3Planes = 15;
+// operand planes of the 3-D right-hand side, f in (b, ux, uy, uz)
+//   z-grid: f value, 4+f dz f;   y-padded: 0 ux, 1 uy, 2 uz, 3+f dy f, 7+f dz f, 11 b
+// dy f is formed where the values enter the y transform, dx f where they enter the x transform: 8
+// and 12 planes pass through memory for the products' 15 operands.
+// Against 15 planes of both kinds, 256 x 256 x 128, FP32 / FP64 us: k3_zbwd 233 / 428 -> 196 / 337,
+// k3_ybwd 365 / 622 -> 312 / 550, k3_xpass 341 / 740 -> 335 / 725.
+constexpr int kCh3ZPlanes = 8;
+constexpr int kCh3Planes = 12;
 
 template <typename T, int NT, int QT = ZbwdTile<T>::QT>
 __global__ __launch_bounds__(NT, 768 / NT) void k3_zbwd(const cplx<T>* __restrict__ b, const cplx<T>* __restrict__ ux,
@@ -35,7 +40,9 @@ __global__ __launch_bounds__(NT, 768 / NT) void k3_zbwd(const cplx<T>* __restric
 // ---------------------------------------------------------------------------
 // k3_ybwd: padded inverse y transform of TK kx-lines of one z level and plane.
 // grid (ceil(nxh/TK), N, planes), remapped so that the tiles of one row of kx (which
-// share cache lines: rows of nxh values are not line-aligned) run on one XCD.
+// share cache lines: rows of nxh values are not line-aligned) run on one XCD, with the
+// value and dy tiles of a row one after the other: the second reads the row from L2.
+// On the kx = 0 and kx = Nx/2 lines dy vanishes at the y Nyquist.
 // ---------------------------------------------------------------------------
 template <typename T, int NY, int MY, int TK, int NT>
 __global__ __launch_bounds__(NT) void k3_ybwd(const cplx<T>* __restrict__ G, Ch3Geom geo, cplx<T>* __restrict__ Q,
@@ -49,10 +56,15 @@ __global__ __launch_bounds__(NT) void k3_ybwd(const cplx<T>* __restrict__ G, Ch3
     if constexpr (TW_LDS) load_twiddles<T, MY, NT>(twl_lds, tw);
     const unsigned gxy = gridDim.x * gridDim.y;
     const unsigned lin = xcd_remap(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gxy * gridDim.z);
-    const int nxh = geo.nxh, z = (int)((lin / gridDim.x) % gridDim.y), pl = (int)(lin / gxy);
-    const int m0 = (int)(lin % gridDim.x) * TK;
+    const int nxh = geo.nxh, m0 = (int)(lin % gridDim.x) * TK;
+    const bool both = lin < 8 * gxy;  // value and dy of a field in turn, then the dz planes
+    const unsigned row = lin / gridDim.x;
+    const int z = (int)((both ? row >> 1 : row) % gridDim.y);
+    const bool dy = both && (row & 1);
+    const int f = (int)(both ? lin / (2 * gxy) : lin / gxy - 8);
+    const int pl = both ? (dy ? 3 + f : (f == 0 ? 11 : f - 1)) : 7 + f;
     const size_t plane = (size_t)geo.N * geo.nmodes;
-    const V* in = G + (size_t)pl * plane + (size_t)z * geo.nmodes;
+    const V* in = G + (size_t)(both ? f : 4 + f) * plane + (size_t)z * geo.nmodes;
     const bool xeven = (geo.nx % 2) == 0;
     cplx<T>* out = Q + (size_t)pl * geo.N * MY * nxh + (size_t)z * MY * nxh;
     // padded position j: ky = j below NY/2, the Nyquist row halved at j = NY/2 and
@@ -66,7 +78,11 @@ __global__ __launch_bounds__(NT) void k3_ybwd(const cplx<T>* __restrict__ G, Ch3
         else if (j > MY - NY / 2) n = NY - MY + j;
         else return V{T(0), T(0)};
         if (m >= nxh) return V{T(0), T(0)};
-        const V v = in[(size_t)n * nxh + m];
+        V v = in[(size_t)n * nxh + m];
+        if (dy) {  // workgroup-uniform
+            const T ky = half && (m == 0 || (xeven && m == geo.nx / 2)) ? T(0) : T(ch3_ky(geo, n));
+            v = V{-ky * v.y, ky * v.x};
+        }
         return half ? V{v.x * T(0.5), v.y * T(0.5)} : v;
     };
     auto store = [&](int c, int j, V v) {
@@ -79,13 +95,13 @@ __global__ __launch_bounds__(NT) void k3_ybwd(const cplx<T>* __restrict__ G, Ch3
 }
 
 // ---------------------------------------------------------------------------
-// k3_xpass: one padded row (z, j) per workgroup: 15 operand rows packed two per
-// complex line (8 lines), inverse x FFT, the four advection products, two forward
-// x FFTs.  Output: four rows of nxh values (scaled by `scale`).
+// k3_xpass: one padded row (z, j) per workgroup: 15 operand rows, dx f = i kx f formed from the
+// value rows, packed two per complex line (8 lines), inverse x FFT, the four advection
+// products, two forward x FFTs.  Output: four rows of nxh values (scaled by `scale`).
 //   F_b  = -(ux dx b  + uy dy b  + uz dz b)   (and likewise F_ux, F_uy, F_uz)
 // ---------------------------------------------------------------------------
 template <typename T, int NX, int MX, int NT>
-__global__ __launch_bounds__(NT) void k3_xpass(const cplx<T>* __restrict__ Q, int N, int MY, T scale,
+__global__ __launch_bounds__(NT) void k3_xpass(const cplx<T>* __restrict__ Q, int N, int MY, double k0x, T scale,
                                                cplx<T>* __restrict__ H, const cplx<T>* __restrict__ tw) {
     using V = cplx<T>;
     constexpr int NXH = NX / 2 + 1;
@@ -98,30 +114,34 @@ __global__ __launch_bounds__(NT) void k3_xpass(const cplx<T>* __restrict__ Q, in
     if constexpr (TW_LDS) load_twiddles<T, MX, NT>(twl_lds, tw);
     const size_t row = (size_t)blockIdx.y * MY + blockIdx.x;  // (z, j)
     const size_t plane = (size_t)N * MY * NXH;
-    // element i of packed line l (planes 2l, 2l+1): a + i b at k = i < NXH (real parts
-    // only at k = 0), conj(a) + i conj(b) at the mirror i = MX - k, zero in between
+    // element i of packed line l: a + i b at k = i < NXH (real parts only at k = 0), conj(a) + i conj(b) at the
+    // mirror i = MX - k, zero in between.  Lines 0..5 hold planes (2l, 2l+1), 6 and 7 the x derivatives of
+    // (b, ux) and (uy, uz): i kx (a + i b) with the mirror's kx negative, zero on the kx = Nx/2 line
     auto load = [&](int line, int i) -> V {
         const bool mirror = i > MX - NXH;
         if (i >= NXH && !mirror) return V{T(0), T(0)};
         const int k = mirror ? MX - i : i;
         const size_t off = row * NXH + k;
-        const V a = Q[(size_t)(2 * line) * plane + off];
-        const V bb = (2 * line + 1 < kCh3Planes) ? Q[(size_t)(2 * line + 1) * plane + off] : V{T(0), T(0)};
-        if (k == 0) return V{a.x, bb.x};
-        return mirror ? V{a.x + bb.y, bb.x - a.y} : V{a.x - bb.y, a.y + bb.x};
+        const bool dx = line >= 6;
+        const V a = Q[(size_t)(dx ? 71 - 10 * line : 2 * line) * plane + off];
+        V bb = Q[(size_t)(dx ? 2 * line - 12 : 2 * line + 1) * plane + off];
+        if (line == 5) bb = V{T(0), T(0)};
+        const V p = k == 0 ? V{a.x, bb.x} : (mirror ? V{a.x + bb.y, bb.x - a.y} : V{a.x - bb.y, a.y + bb.x});
+        const T kx = 2 * k == NX ? T(0) : T(k0x * (mirror ? -k : k));
+        return V{dx ? -kx * p.y : p.x, dx ? kx * p.x : p.y};  // selects: a thread's loads stay in flight together
     };
     fft_regs_io<T, MX, NL, NT, true, false, true, false>(buf, twl, load, [](int, int, V) {});  // lines are rows
-    // line l holds planes (2l, 2l+1): l0 = (ux, uy), l1 = (uz, dx b), l2 = (dy b, dz b),
-    // l3 = (dx ux, dy ux), l4 = (dz ux, dx uy), l5 = (dy uy, dz uy), l6 = (dx uz, dy uz), l7 = (dz uz, 0)
+    // l0 = (ux, uy), l1 = (uz, dy b), l2 = (dy ux, dy uy), l3 = (dy uz, dz b), l4 = (dz ux, dz uy),
+    // l5 = (dz uz, 0), l6 = (dx b, dx ux), l7 = (dx uy, dx uz)
     for (int x = threadIdx.x; x < MX; x += NT) {
         const V l0 = buf[0 * LS + pidx(x)], l1 = buf[1 * LS + pidx(x)], l2 = buf[2 * LS + pidx(x)];
         const V l3 = buf[3 * LS + pidx(x)], l4 = buf[4 * LS + pidx(x)], l5 = buf[5 * LS + pidx(x)];
         const V l6 = buf[6 * LS + pidx(x)], l7 = buf[7 * LS + pidx(x)];
         const T vx = l0.x, vy = l0.y, vz = l1.x;
-        const T fb = -(vx * l1.y + vy * l2.x + vz * l2.y) * scale;
-        const T fux = -(vx * l3.x + vy * l3.y + vz * l4.x) * scale;
-        const T fuy = -(vx * l4.y + vy * l5.x + vz * l5.y) * scale;
-        const T fuz = -(vx * l6.x + vy * l6.y + vz * l7.x) * scale;
+        const T fb = -(vx * l6.x + vy * l1.y + vz * l3.y) * scale;
+        const T fux = -(vx * l6.y + vy * l2.x + vz * l4.x) * scale;
+        const T fuy = -(vx * l7.x + vy * l2.y + vz * l4.y) * scale;
+        const T fuz = -(vx * l7.y + vy * l3.x + vz * l5.x) * scale;
         // each thread reads and rewrites only its own x positions: no barrier needed here
         buf[0 * LS + pidx(x)] = V{fb, fux};
         buf[1 * LS + pidx(x)] = V{fuy, fuz};

@@ -88,7 +88,7 @@ Channel3Solver::Channel3Solver(Context* ctx, const Channel3Desc& d) : ctx_(ctx),
         }
     }
     const size_t prow = (size_t)d.nz * my_ * nxh_ * vb;  // one y-padded plane
-    G_ = DevBuf(ctx_, (size_t)kCh3Planes * fb);
+    G_ = DevBuf(ctx_, (size_t)kCh3ZPlanes * fb);
     Q_ = DevBuf(ctx_, (size_t)kCh3Planes * prow);
     H_ = DevBuf(ctx_, (size_t)4 * prow);
     // Chebyshev tables
@@ -383,7 +383,8 @@ void Channel3Solver::rhs_t(void* F0, void* F1, void* F2, void* F3) {
             const V* tw = static_cast<const V*>(ctx_->twiddle(MX, dt));
             constexpr int NT = NX >= 512 ? 512 : 256;
             timed(2, [&] {
-                hipLaunchKernelGGL((k3_xpass<T, NX, MX, NT>), dim3(my_, N), dim3(NT), 0, s, Q, N, my_, scale, H, tw);
+                hipLaunchKernelGGL((k3_xpass<T, NX, MX, NT>), dim3(my_, N), dim3(NT), 0, s, Q, N, my_, geo.k0x, scale,
+                                   H, tw);
             });
         } else {
             TG_REQUIRE(false, kErrInvalid, "3-D channel solver: x size too large for this dtype");
@@ -683,9 +684,9 @@ void Channel3Solver::kernel_bytes(double* out) const {
     const double vb = 2.0 * dtype_size((DType)d_.dtype), rb = dtype_size((DType)d_.dtype);
     const double nc = (double)nmodes_ * d_.nz, N = d_.nz;
     const double pad = (double)d_.nz * my_ * nxh_;
-    out[0] = (4 * nc + kCh3Planes * nc) * vb + 2 * N * N * rb;  // read 4 fields, write 15 planes
-    out[1] = (kCh3Planes * nc + kCh3Planes * pad) * vb;         // read 15 planes, write 15 y-padded planes
-    out[2] = (kCh3Planes * pad + 4 * pad) * vb;                 // read 15 padded planes, write 4
+    out[0] = (4 * nc + kCh3ZPlanes * nc) * vb + 2 * N * N * rb;  // read 4 fields, write 8 planes
+    out[1] = (kCh3ZPlanes * nc + kCh3Planes * pad) * vb;        // read 8 planes, write 12 y-padded planes
+    out[2] = (kCh3Planes * pad + 4 * pad) * vb;                 // read 12 padded planes, write 4
     out[3] = (4 * pad + 4 * nc) * vb;                           // read 4 padded planes, write 4
     out[4] = (8 * nc) * vb + N * N * rb;                        // read 4 planes, write 4 rows
     out[5] = (4 * 4 + 4 + 5) * nc * vb;                         // state (x2 on the kx lines), F, histories, rhs
@@ -709,7 +710,7 @@ size_t footprint(const Channel3Desc& d) {
     const size_t nfields = 5 + 12 + 5 + (ms ? 0 : 4 + 9 * S);  // state, history, rhs rows, RK stage rows
     // distinct |k_h|^2 keys: at most one per mode (about nmodes / 5.6 at 256 x 256 when Lx == Ly)
     const size_t keys = d.Lx == d.Ly ? nmodes / 3 + 64 : nmodes;
-    size_t b = nfields * alloc_granule(fb) + alloc_granule(kCh3Planes * fb) + alloc_granule(kCh3Planes * prow) +
+    size_t b = nfields * alloc_granule(fb) + alloc_granule(kCh3ZPlanes * fb) + alloc_granule(kCh3Planes * prow) +
                alloc_granule(4 * prow);                                                           // G, Q, H
     b += alloc_granule(nmodes * kCh3TauStride * vb) + 3 * alloc_granule(N * N * ib);           // taus, tables
     b += alloc_granule(tau_table_doubles(tau_shape(d.nz, true), keys) * sizeof(double));  // tau-solve tables

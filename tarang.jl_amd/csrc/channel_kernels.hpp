@@ -92,10 +92,10 @@ __host__ __device__ inline double ch3_ky(const Ch3Geom& g, int n) {
 // the next pass) with every column tile, both products and both parities, its loads one
 // batch ahead of its products.  A lane then holds Re and Im of one mode and writes whole
 // complex values straight to the z-major planes (16 consecutive modes per row).
-// Derived planes: dx f = i kx value, dy f = i ky value.  On the kx = 0 and kx = Nx/2
-// lines the projected state's x derivative vanishes, and so does its y derivative at
-// the y Nyquist; the kx = Nx/2 line is halved.  2-D: eight planes (no y), and the kx = 0
-// and kx = Nx/2 lines keep only their real part (the grid round trip of the state).
+// The kx = Nx/2 line is halved.  3-D: eight planes, value (b, ux, uy, uz) and dz; the y
+// and x passes form dy and dx from the values.  2-D: eight planes, dx f = i kx value among
+// them (zero on the kx = 0 and kx = Nx/2 lines, where the projected state's x derivative
+// vanishes), and those lines keep only their real part (the grid round trip of the state).
 // ---------------------------------------------------------------------------
 // modes per workgroup (QT, a multiple of 16), k steps per load batch (U) and threads per
 // workgroup (NT)
@@ -134,23 +134,21 @@ __device__ inline void zbwd_mfma(const cplx<T>* __restrict__ b, const cplx<T>* _
     const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t plane = (size_t)N * nmodes;
-    const bool xeven = (geo.nx % 2) == 0, yeven = (geo.ny % 2) == 0;
-    // per mode group: this lane's mode and its derivative factors
-    T kxv[NG], kyv[NG], wv[NG];
-    bool dxz[NG], dyz[NG], live[NG];
+    const bool xeven = (geo.nx % 2) == 0;
+    // per mode group: this lane's mode and its factors
+    T kxv[NG], wv[NG];
+    bool xline[NG], live[NG];
     int qq[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
         const int q = q0 + 16 * g + r16;
         qq[g] = q;
         live[g] = q < nmodes;
-        const int m = q % geo.nxh, n = q / geo.nxh;
-        const bool xny = xeven && m == geo.nx / 2, xline = m == 0 || xny;
+        const int m = q % geo.nxh;
+        const bool xny = xeven && m == geo.nx / 2;
         kxv[g] = T(geo.k0x * m);
-        kyv[g] = T(ch3_ky(geo, n));
         wv[g] = xny ? T(0.5) : T(1);
-        dxz[g] = xline;
-        dyz[g] = xline && yeven && n == geo.ny / 2;
+        xline[g] = m == 0 || xny;
     }
     // first-half z tiles of this workgroup: all, or a share when the grid splits z (blockIdx.z)
     const int zper = (nzh + (int)gridDim.z - 1) / (int)gridDim.z;
@@ -210,21 +208,18 @@ __device__ inline void zbwd_mfma(const cplx<T>* __restrict__ b, const cplx<T>* _
             multiply(sb + U, amB, bvB);
         }
         auto put = [&](int zz, int g, V val, V dzv) {
-            const V dx = dxz[g] ? V{T(0), T(0)} : V{-kxv[g] * val.y, kxv[g] * val.x};  // i kx v
             const size_t o = (size_t)zz * nmodes + qq[g];
             if constexpr (TWO_D) {
+                const V dx = xline[g] ? V{T(0), T(0)} : V{-kxv[g] * val.y, kxv[g] * val.x};  // i kx v
                 // no y transform follows: the kx = 0 and kx = Nx/2 lines keep their real part here
-                if (dxz[g]) val.y = dzv.y = T(0);
+                if (xline[g]) val.y = dzv.y = T(0);
                 // planes 0 ux, 1 uz, 2 dx b, 3 dz b, 4 dx ux, 5 dz ux, 6 dx uz, 7 dz uz
                 if (f > 0) G[(size_t)(f - 1) * plane + o] = val;
                 G[(size_t)(2 + 2 * f) * plane + o] = dx;
                 G[(size_t)(3 + 2 * f) * plane + o] = dzv;
             } else {
-                const V dy = dyz[g] ? V{T(0), T(0)} : V{-kyv[g] * val.y, kyv[g] * val.x};
-                if (f > 0) G[(size_t)(f - 1) * plane + o] = val;  // ux, uy, uz
-                G[(size_t)(3 + 3 * f) * plane + o] = dx;
-                G[(size_t)(4 + 3 * f) * plane + o] = dy;
-                G[(size_t)(5 + 3 * f) * plane + o] = dzv;
+                G[(size_t)f * plane + o] = val;
+                G[(size_t)(4 + f) * plane + o] = dzv;
             }
         };
 #pragma unroll
