@@ -361,7 +361,7 @@ template <typename T>
 struct Ch3StageArgs {
     const cplx<T>* X0[4];      // b, ux, uy, uz at the start of the step
     const cplx<T>* F[4][4];    // F_j rows E2, E3x, E3y, E3z
-    const cplx<T>* LX[4][5];   // LX_j rows E1..E3z
+    const cplx<T>* LX[4][5];   // LX_j rows E1..E3z (null: no weight in this stage)
     T ae[4], ai[4];
     int nterms;
     T dt;
@@ -381,9 +381,11 @@ __global__ void k3_stage(Ch3StageArgs<T> a, size_t n) {
                     v.x += a.dt * a.ae[j] * f.x;
                     v.y += a.dt * a.ae[j] * f.y;
                 }
-                const cplx<T> l = a.LX[j][r][i];
-                v.x -= a.dt * a.ai[j] * l.x;
-                v.y -= a.dt * a.ai[j] * l.y;
+                if (a.LX[j][r]) {
+                    const cplx<T> l = a.LX[j][r][i];
+                    v.x -= a.dt * a.ai[j] * l.x;
+                    v.y -= a.dt * a.ai[j] * l.y;
+                }
             }
             a.out[a.final_update ? r - 1 : r][i] = v;
         }

@@ -514,9 +514,10 @@ void Channel3Solver::stage_t(int st, bool final_update) {
     const int nterms = final_update ? tab_.stages : st;
     for (int j = 0; j < nterms; ++j) {
         for (int r = 0; r < 4; ++r) a.F[j][r] = Frk_[j][r].as<const V>();
-        for (int r = 0; r < 5; ++r) a.LX[j][r] = LX_[j][r].as<const V>();
+        const double ai = final_update ? tab_.bI[j] : tab_.AI[st][j];
+        for (int r = 0; r < 5; ++r) a.LX[j][r] = ai != 0.0 ? LX_[j][r].as<const V>() : nullptr;
         a.ae[j] = T(final_update ? tab_.bE[j] : tab_.AE[st][j]);
-        a.ai[j] = T(final_update ? tab_.bI[j] : tab_.AI[st][j]);
+        a.ai[j] = T(ai);
     }
     a.nterms = nterms;
     a.dt = T(d_.dt);
@@ -560,12 +561,12 @@ void Channel3Solver::launch_step_body() {
                                        r == 2 ? TAU_.as<V>() : nullptr, r == 2 ? (size_t)nmodes_ * kCh3TauStride : 0);
                 });
             rhs_t<T>(Frk_[0][0].ptr, Frk_[0][1].ptr, Frk_[0][2].ptr, Frk_[0][3].ptr);
-            lx_t<T>(0);
+            if (uses_lx(tab_, 0)) lx_t<T>(0);
             for (int st = 1; st < tab_.stages; ++st) {
                 stage_t<T>(st, false);
                 solve_t<T>();
                 rhs_t<T>(Frk_[st][0].ptr, Frk_[st][1].ptr, Frk_[st][2].ptr, Frk_[st][3].ptr);
-                lx_t<T>(st);
+                if (uses_lx(tab_, st)) lx_t<T>(st);
             }
             stage_t<T>(0, true);
             zero_t<T>(P_.ptr, n);

@@ -300,9 +300,10 @@ void ChannelSolver::stage_rhs_t(int st, bool final_update) {
     const int nterms = final_update ? tab_.stages : st;
     for (int j = 0; j < nterms; ++j) {
         for (int r = 0; r < 3; ++r) a.F[j][r] = F_[j][r].as<const V>();
-        for (int r = 0; r < 4; ++r) a.LX[j][r] = LX_[j][r].as<const V>();
+        const double ai = final_update ? tab_.bI[j] : tab_.AI[st][j];
+        for (int r = 0; r < 4; ++r) a.LX[j][r] = ai != 0.0 ? LX_[j][r].as<const V>() : nullptr;
         a.ae[j] = T(final_update ? tab_.bE[j] : tab_.AE[st][j]);
-        a.ai[j] = T(final_update ? tab_.bI[j] : tab_.AI[st][j]);
+        a.ai[j] = T(ai);
     }
     a.nterms = nterms;
     a.dt = T(d_.dt);
@@ -417,7 +418,7 @@ void ChannelSolver::zero_t(void* p, size_t n) {
 
 // The launches between implicit solves i - 1 and i of a step (i = nsolves(): after the last)
 //   multistep: [F_n, SBDF right-hand side] solve []
-//   RK:        [X0 copy, p = taus = 0, F_0, L x_0, stage-1 rhs] solve [F_1, L x_1, stage-2 rhs]
+//   RK:        [X0 copy, p = taus = 0, F_0, stage-1 rhs] solve [F_1, L x_1, stage-2 rhs]
 //              solve ... [F_{s-1}, L x_{s-1}, final update, p = taus = 0]
 template <typename T>
 void ChannelSolver::segment_t(int i) {
@@ -442,7 +443,7 @@ void ChannelSolver::segment_t(int i) {
         TG_HIP(hipGetLastError());
     }
     rhs_t<T>(B_.ptr, UX_.ptr, UZ_.ptr, F_[i][0].ptr, F_[i][1].ptr, F_[i][2].ptr);
-    lx_t<T>(i);
+    if (uses_lx(tab_, i)) lx_t<T>(i);
     if (i + 1 < tab_.stages) {
         stage_rhs_t<T>(i + 1, false);
     } else {

@@ -15,6 +15,13 @@ struct Tableau {
     int stages = 0;
     double AE[4][4] = {}, AI[4][4] = {}, bE[4] = {}, bI[4] = {}, c[4] = {};
 };
+// whether L x_j has a weight in a later stage or in the update (the first column of the implicit
+// tableaus is zero: L x_0 is never read)
+inline bool uses_lx(const Tableau& t, int j) {
+    bool any = t.bI[j] != 0.0;
+    for (int s = j + 1; s < t.stages; ++s) any = any || t.AI[s][j] != 0.0;
+    return any;
+}
 Tableau make_tableau(int stepper);
 bool is_multistep(int stepper);
 
