@@ -122,13 +122,28 @@ __device__ inline void zbwd_mfma(const cplx<T>* __restrict__ b, const cplx<T>* _
     const int KP = (N + 15) & ~15, NH = (N + 1) / 2, nzh = zbwd_half_tiles(N);
     const int f = blockIdx.y, q0 = blockIdx.x * QT;
     const V* in = f == 0 ? b : (f == 1 ? ux : (f == 2 && !TWO_D ? uy : uz));
-    for (int idx = threadIdx.x; idx < QT * KP; idx += NT) {
-        const int q = idx / KP, k = idx - q * KP;
-        V v{T(0), T(0)};
-        if (q0 + q < nmodes && k < N) v = in[(size_t)(q0 + q) * N + k];
-        const int col = 32 * (q >> 4) + (q & 15);
-        C[k * S + col] = v.x;
-        C[k * S + col + 16] = v.y;
+    // eight loads in flight per thread: one at a time, each turn waited for memory (3-D 256 x 256 x 128: 196 / 337 us
+    // in FP32 / FP64 against 152 / 263; 2-D 1024 x 256 FP32 24.6 against 22.3, 320 x 97 FP64 14.0 against 12.4)
+    constexpr int FB = 8;
+    for (int i0 = threadIdx.x; i0 < QT * KP; i0 += FB * NT) {
+        T re[FB], im[FB];
+#pragma unroll
+        for (int u = 0; u < FB; ++u) {
+            const int idx = i0 + u * NT, q = idx / KP, k = idx - q * KP;
+            const bool ok = q < QT && q0 + q < nmodes && k < N;
+            const V v = in[ok ? (size_t)(q0 + q) * N + k : 0];
+            re[u] = ok ? v.x : T(0);
+            im[u] = ok ? v.y : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < FB; ++u) {
+            const int idx = i0 + u * NT, q = idx / KP, k = idx - q * KP;
+            const int col = 32 * (q >> 4) + (q & 15);
+            if (q < QT) {
+                C[k * S + col] = re[u];
+                C[k * S + col + 16] = im[u];
+            }
+        }
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
@@ -380,24 +395,37 @@ __global__ __launch_bounds__(NT, 768 / NT) void k_ch_zfwd(const cplx<T>* __restr
     const int ke = kb + kps < nkt ? kb + kps : nkt;
     const V* in = H + (size_t)f * N * nmodes;
     const bool xeven = (nx % 2) == 0;
-    for (int idx = threadIdx.x; idx < QT * NHP; idx += NT) {
-        const int zz = idx / QT, q = idx - zz * QT;
-        const int m = q0 + q, zm = N - 1 - zz;
-        V hz{T(0), T(0)}, hm{T(0), T(0)};
-        if (zz < NH && m < nmodes) {
-            hz = in[(size_t)zz * nmodes + m];
-            if (zm != zz) hm = in[(size_t)zm * nmodes + m];
+    // four rows in flight per thread: one at a time, each turn waited for memory (3-D 256 x 256 x 128: 114 / 180 us
+    // in FP32 / FP64 against 109 / 165)
+    constexpr int FB = 4;
+    for (int i0 = threadIdx.x; i0 < QT * NHP; i0 += FB * NT) {
+        T zr[FB], zi[FB], mr[FB], mi[FB];
+#pragma unroll
+        for (int u = 0; u < FB; ++u) {
+            const int idx = i0 + u * NT, zz = idx / QT, m = q0 + idx - zz * QT, zm = N - 1 - zz;
+            const bool ok = zz < NH && m < nmodes, two = ok && zm != zz;
+            const V hz = in[ok ? (size_t)zz * nmodes + m : 0], hm = in[two ? (size_t)zm * nmodes + m : 0];
+            zr[u] = ok ? hz.x : T(0);
+            zi[u] = ok ? hz.y : T(0);
+            mr[u] = two ? hm.x : T(0);
+            mi[u] = two ? hm.y : T(0);
         }
-        if (xeven && m == nx / 2) {
-            hz = V{T(2) * hz.x, T(0)};
-            hm = V{T(2) * hm.x, T(0)};
+#pragma unroll
+        for (int u = 0; u < FB; ++u) {
+            const int idx = i0 + u * NT, zz = idx / QT, q = idx - zz * QT;
+            if (zz >= NHP) continue;
+            V hz{zr[u], zi[u]}, hm{mr[u], mi[u]};
+            if (xeven && q0 + q == nx / 2) {
+                hz = V{T(2) * hz.x, T(0)};
+                hm = V{T(2) * hm.x, T(0)};
+            }
+            const int col = 32 * (q >> 4) + (q & 15);
+            const bool mid = N - 1 - zz == zz;  // the middle point (N odd) counts once, in the even sums
+            CS[zz * S + col] = hz.x + hm.x;
+            CS[zz * S + col + 16] = hz.y + hm.y;
+            CA[zz * S + col] = mid ? T(0) : hz.x - hm.x;
+            CA[zz * S + col + 16] = mid ? T(0) : hz.y - hm.y;
         }
-        const int col = 32 * (q >> 4) + (q & 15);
-        const bool mid = zm == zz;  // the middle point (N odd) counts once, in the even sums
-        CS[zz * S + col] = hz.x + hm.x;
-        CS[zz * S + col + 16] = hz.y + hm.y;
-        CA[zz * S + col] = mid ? T(0) : hz.x - hm.x;
-        CA[zz * S + col + 16] = mid ? T(0) : hz.y - hm.y;
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
