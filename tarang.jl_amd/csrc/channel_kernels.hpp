@@ -97,10 +97,17 @@ __host__ __device__ inline double ch3_ky(const Ch3Geom& g, int n) {
 // them (zero on the kx = 0 and kx = Nx/2 lines, where the projected state's x derivative
 // vanishes), and those lines keep only their real part (the grid round trip of the state).
 // ---------------------------------------------------------------------------
-// modes per workgroup (QT, a multiple of 16), k steps per load batch (U) and threads per
-// workgroup (NT)
-template <typename T> struct ZbwdTile { static constexpr int QT = 32, U = 4, NT = 256; };
-template <> struct ZbwdTile<double> { static constexpr int QT = 16, U = 2, NT = 256; };
+// modes per workgroup (QT, a multiple of 16), threads per workgroup (NT) and k steps per load batch
+// of a tile of qt modes: eight for the FP32 tiles of 16 that the few modes of a 2-D problem take, a round
+// trip to L2 per batch (1024 x 256: 19.9 us, four steps 22.3); FP64 loses registers by four (3-D 281 us, two 263)
+template <typename T> struct ZbwdTile {
+    static constexpr int QT = 32, NT = 256;
+    static constexpr int steps(int qt) { return qt == 16 ? 8 : 4; }
+};
+template <> struct ZbwdTile<double> {
+    static constexpr int QT = 16, NT = 256;
+    static constexpr int steps(int) { return 2; }
+};
 
 __host__ __device__ inline int zbwd_lds_stride(int qt) { return 2 * qt + 1; }
 // first-half z tiles of the parity-split evaluation
@@ -115,7 +122,7 @@ __device__ inline void zbwd_mfma(const cplx<T>* __restrict__ b, const cplx<T>* _
     using acc4 = typename Op::acc4;
     using V = cplx<T>;
     constexpr int NG = QT / 16, CT = 2 * NG, S = 2 * QT + 1;
-    constexpr int U = ZbwdTile<T>::U, NWV = NT / 64;
+    constexpr int U = ZbwdTile<T>::steps(QT), NWV = NT / 64;
     extern __shared__ unsigned char smem_raw[];
     T* C = reinterpret_cast<T*>(smem_raw);  // [KP][S]
     const int N = geo.N, nmodes = geo.nmodes;
