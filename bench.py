@@ -113,7 +113,7 @@ def main():
     ap.add_argument("--requests", type=int, default=24, help="serving: number of requests")
     ap.add_argument("--cfl-horizon", action="store_true",
                     help="channel: also run the configuration to its t = 20 horizon with CFL-controlled dt "
-                         "(FP64 and FP32 split-inverse forms through the API)")
+                         "(FP64 and FP32 state through the API)")
     ap.add_argument("--no-group", action="store_true",
                     help="channel: skip the group-stepping comparison (used for profiler runs)")
     ap.add_argument("--cfl-wall", type=float, default=480.0,
@@ -310,7 +310,7 @@ CH_KERNELS = ["k_ch_zbwd (Chebyshev evaluation of 8 operand planes)",
               "k_ch_xpass (inverse x FFTs M=1536, products, forward x FFTs)",
               "k_ch_zfwd (Chebyshev forward of 3 products)",
               "k_ch_lx (structured L x per mode)",
-              "k_ch_solve (per-mode explicit inverses, FP64 GEMV, parity-split systems)",
+              "k_ch_tau_solve (per-mode tridiagonal tau lines, FP64, parity-split)",
               "stage / copy / zero"]
 
 
@@ -339,9 +339,8 @@ def dt_change_cost(_lib, ctx, h, pre, dt, steady_ms):
     return {"ms_of_the_3_steps_after_a_change": out, "steady_ms_per_step": steady_ms}
 
 
-# FP32 forms of the channel solvers: (name, refine_sweeps, split_inverse); the first is the
-# headline form.  split_inverse stores every tau-system inverse entry as an FP32 value plus a
-# 8-bit remainder (2^-32 relative); refine_sweeps adds FP64-residual refinement sweeps.
+# FP32 settings of the channel solvers: (name, refine_sweeps, split_inverse); the first is the
+# headline form.  The solves are direct and in FP64, so all four do the same work.
 FP32_FORMS = (("f32", 0, 1), ("f32_plain", 0, 0), ("f32_sweeps1", 1, 0), ("f32_sweeps2", 2, 0))
 FP32_HEADLINE = {"refine_sweeps": FP32_FORMS[0][1], "split_inverse": FP32_FORMS[0][2]}
 
@@ -495,7 +494,7 @@ def bench_channel(a):
     return line
 
 
-# a group of uneven 2-D channel problems (nx, nz, Ra): FP32 split inverses, RK222, dt = 1e-3
+# a group of uneven 2-D channel problems (nx, nz, Ra): FP32 state, RK222, dt = 1e-3
 GROUP_MEMBERS = [(256, 64, 1e6)] * 4 + [(512, 128, 2e6)] * 4 + [(1024, 64, 5e5)] * 2 + [(128, 256, 1e7)] * 2
 
 
@@ -572,7 +571,7 @@ def channel_group_bench(a):
             _lib.call("tarang_chan_destroy", h)
     _lib.call("tarang_ctx_destroy", ctx)
     return {"members": [{"nx": nx, "nz": nz, "Ra": Ra} for nx, nz, Ra in GROUP_MEMBERS],
-            "form": "FP32 split inverses, RK222, dt = 1e-3", "steps": steps, "alone": out["alone"],
+            "form": "FP32 state, RK222, dt = 1e-3", "steps": steps, "alone": out["alone"],
             "group": out["group"], "speedup": out["alone"]["ms_per_step"] / out["group"]["ms_per_step"],
             "same_bits": same}
 
@@ -580,7 +579,7 @@ def channel_group_bench(a):
 def channel_cfl_horizon(a):
     """The 2-D configuration run to its horizon t = 20 (2000 steps of the fixed dt = 0.01 at
     most) with the CFL controller choosing dt (max_dt = 0.01, safety 0.5, cadence 10), FP64
-    and the FP32 split-inverse form, through the API mirror.  Convection at Ra = 2e6 is
+    and the FP32 form, through the API mirror.  Convection at Ra = 2e6 is
     chaotic, so the two trajectories decorrelate: they are compared by the time-averaged
     Nusselt number over t in [10, 20], not pointwise."""
     import numpy as np
@@ -651,11 +650,11 @@ def channel_cfl_horizon(a):
 CH3 = dict(nx=256, ny=256, nz=128, Lx=4.0, Ly=4.0, Lz=1.0, Ra=1e7, Pr=0.7, dt=2e-3)
 CH3_WORKLOAD = ("3-D Rayleigh-Benard, RealFourier^2 x ChebyshevT 256x256x128, Lx=Ly=4, Lz=1, Ra=1e7, Pr=0.7, "
                 "no-slip walls, b fixed at both walls, 3/2 dealiasing, SBDF2, dt=2e-3")
-CH3_KERNELS = ["k3_zbwd (Chebyshev evaluation of 15 operand planes)", "k3_ybwd (padded inverse y FFT, MY=384)",
+CH3_KERNELS = ["k3_zbwd (Chebyshev evaluation of 8 operand planes)", "k3_ybwd (padded inverse y FFT, MY=384)",
                "k3_xpass (inverse x FFTs MX=384, 12 products, forward x FFTs)",
                "k3_yfwd (forward y FFT, truncation, Nyquist folds)", "k_ch_zfwd (Chebyshev forward of 4 products)",
                "k3_sbdf (multistep right-hand side)",
-               "k3_solve (explicit inverses per k_h^2 key, 8-mode chunks on FP64 matrix cores)",
+               "k3_tau_solve (per-mode tridiagonal tau lines, FP64)",
                "k3_lx (structured L x, RK only)"]
 
 
@@ -807,8 +806,8 @@ def bench_channel3d(a):
 SERVE_WORKLOAD = ("serving stream: Poisson arrivals at 80% of the measured saturation capacity; 40% 2-D turbulence "
                   "N in {128,256,512,1024}^2 (RK443, dt=1e-3), 40% 2-D Rayleigh-Benard Nx x Nz in {128x32, 256x64, "
                   "512x128, 1024x256}, Ra log-uniform in [1e5, 1e8], Pr=1 (RK222, dt=1e-3), 20% 1-D Burgers N in "
-                  "{64..4096}, nu=1e-2 (RK222, dt=1e-3); FP32 state, FP64 tau factorisation, inverses stored as FP32 "
-                  "values plus 8-bit remainders; steps log-uniform in [200, 2000]")
+                  "{64..4096}, nu=1e-2 (RK222, dt=1e-3); FP32 state, direct FP64 tau "
+                  "solves; steps log-uniform in [200, 2000]")
 
 
 def serving_stream(np, torch, _lib, configs, n, seed, dev):
@@ -836,7 +835,7 @@ def serving_stream(np, torch, _lib, configs, n, seed, dev):
             d = _lib.ChanDesc()
             d.nx, d.nz, d.Lx, d.Lz, d.kappa, d.nu, d.dt = nx, nz, 4.0, 1.0, Ra ** -0.5, Ra ** -0.5, 1e-3
             d.dtype, d.timestepper, d.b_bottom, d.b_top = _lib.F32, 0, 1.0, 0.0
-            d.refine_sweeps = FP32_HEADLINE["refine_sweeps"]  # FP32 state, refined tau inverses
+            d.refine_sweeps = FP32_HEADLINE["refine_sweeps"]  # FP32 state
             d.split_inverse = FP32_HEADLINE["split_inverse"]
             bg, _ = channel_ic(np, nx, nz, 1.0, seed=int(rng.integers(1 << 30)))
             k = np.arange(nz)
