@@ -277,7 +277,7 @@ class _ChannelBackend:
         d.dt = solver.dt
         d.dtype = _lib.F32 if dom.dtype == np.float32 else _lib.F64
         d.timestepper = timestepper.code
-        # the FP32 state's default solve form: inverses with 8-bit remainders (the library
+        # on by default for an FP32 state; the solves are the same either way (the library
         # refuses split_inverse = 1 for an FP64 state, so an explicit request there fails loudly)
         split = (dom.dtype == np.float32) if split_inverse is None else bool(split_inverse)
         d.split_inverse = 1 if split else 0
