@@ -317,8 +317,10 @@ double Channel3Solver::implicit_c(bool first) const {
 }
 
 TauSys Channel3Solver::tau_sys() const {
-    return TauSys{d_.nz, tau_shape(d_.nz, true), nkeys_, factored_c_, 2.0 / d_.Lz, d_.kappa, d_.nu,
-                  kh_.as<const double>(), 0.0, tab_tau_.as<double>()};
+    const bool fp64 = d_.dtype == kF64;
+    const double sz = 2.0 / d_.Lz;
+    return TauSys{d_.nz, tau_shape(d_.nz, true), nkeys_, factored_c_, sz, d_.kappa, d_.nu, kh_.as<const double>(), 0.0,
+                  tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
 }
 
 void Channel3Solver::factor(double c) {
@@ -457,7 +459,7 @@ void Channel3Solver::solve_t() {
     a.bcv = bcv_.as<const double2>();
     a.modes = modes_.as<const int2>();
     a.rot = rot_.as<const double>();
-    a.psi = tau_uses_psi(d_.nz, factored_c_, 2.0 / d_.Lz, d_.kappa, d_.nu, kh_max_);
+    a.psi = tau_uses_psi(a.t, kh_max_);
     a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
     a.R2 = R_[1].as<const V>();
     a.R3x = R_[2].as<const V>();

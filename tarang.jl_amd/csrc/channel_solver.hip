@@ -329,11 +329,12 @@ TauArgs<T> ChannelSolver::solve_args() const {
     using V = cplx<T>;
     TauArgs<T> a{};
     const double k0x = 2.0 * M_PI / d_.Lx, sz = 2.0 / d_.Lz;
+    const bool fp64 = d_.dtype == kF64;
     a.t = TauSys{d_.nz, tau_shape(d_.nz, false), nxh_, factored_c_, sz, d_.kappa, d_.nu, nullptr, k0x,
-                 tab_tau_.as<double>()};
+                 tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
     a.nmodes = nxh_;
     a.bcv = bcv_.as<const double2>();
-    a.psi = tau_uses_psi(d_.nz, factored_c_, sz, d_.kappa, d_.nu, k0x * (nxh_ - 1));
+    a.psi = tau_uses_psi(a.t, k0x * (nxh_ - 1));
     a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
     a.R2 = R_[1].as<const V>();
     a.R3x = R_[2].as<const V>();

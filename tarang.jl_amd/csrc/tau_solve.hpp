@@ -25,7 +25,7 @@
 //      integral alone (t = -1, a = m/(4 (N-1)(N-2))); row N-3 has no upper neighbour
 //   B: D T_{N-1} has the coefficients 2(N-1) (half of it at 0), which B maps to zero below row
 //      N-2, so only row N-2 changes (t = 0, G_{N-1} drops out)
-// Where m >> N^2 (tau_psi_bound) the same recursion runs on psi = m u - r/beta instead, closed by
+// Where m is large (tau_psi_bound) the same recursion runs on psi = m u - r/beta instead, closed by
 // sum psi = m w - sum r/beta: u = (beta psi + r)/alpha then keeps the digits that the second
 // integral would lose.
 //
@@ -35,6 +35,10 @@
 // lambda follows from E1 on the wall, s sum k^2 uz_k + tau_u1z - sum d = 0.  The responses u~_1,
 // uz_1, p_1 depend on (kh, c) only and come from the set-up kernel.  kh = 0 decouples: uz is the
 // integral of E1, p the integral of E3z.
+// At small kh (tau_low_kh) uz is what little the pressure gradient leaves of R3z, so the digits that
+// E3z loses there are those of uz.  E1 keeps them: from degree 1 on uz is the integral of f = d + kh u~
+// (row N - 1: tau_u1z = f_{N-1}), its degree 0 the wall sum, and lambda makes the two agree: for an odd
+// uz the integral's wall sum vanishes, for an even one its degree 0 is that of the E3z line.
 //
 // A solve reads the right-hand-side rows and 6 N doubles per |k_h| key and writes the solution
 // (3-D 256 x 256 x 128: 0.33 GB in FP32); the set-up is one small kernel.
@@ -46,12 +50,18 @@
 
 namespace tarang {
 
-// Where the psi-form starts, as a bound on m.  Against long-double solves the psi-form is exact to
-// rounding from m = N^2 on; the u-form's u_{N-1} loses m/(4 N^2) eps |u_{N-3}|.  Below 64 degrees,
-// where the top degrees may carry weight, the change is at 16 N^2 (a loss of 4 eps); from 64 on at
-// 256 N^2: the psi-form keeps r and a rounding estimate in registers beside the recursion, and the
-// top degrees of a resolved line are small.
-__host__ __device__ inline double tau_psi_bound(int N) { return (N < 64 ? 16.0 : 256.0) * N * N; }
+// Where the psi-form starts, as a bound on |m|.  FP64: at N^2/8, where the two are equally far from a
+// long-double solve (N = 128: 2e-16 and 1e-16 of the line's 2-norm at m = N^2/20, 4e-16 and 1e-16 at
+// 16 N^2, 1e-15 and 2e-16 at 1000 N^2; a dense LU 2e-16).  FP32 rounds the result at 6e-8, and the psi-form
+// keeps r and a rounding estimate in registers beside the recursion: it starts where the u-form's
+// u_{N-1}, which loses m/(4 N^2) eps |u_{N-3}|, would lose 4 eps (64 from 64 degrees on).
+inline double tau_psi_bound(int N, bool fp64) { return (fp64 ? 0.125 : N < 64 ? 16.0 : 256.0) * N * N; }
+// Up to which kh uz is the integral of E1, in units of s; -1: never.  Against long-double solves at N = 128
+// and m = 30 N^2 / 1000 N^2, uz from E3z / from E1 / by a dense inverse is off by 5e-14 / 1e-15 / 1e-15 and
+// 1e-13 / 4e-16 / 2e-15 at kh = 0.8 s, 2e-15 / 7e-16 / 1e-15 at 8 s, 1e-15 / 1e-15 / 1e-15 at 18 s and
+// 5e-16 / 2e-15 / 1e-15 at 50 s: the integral carries kh eps |u~|.  Few degrees bring the line
+// forward.  FP32 rounds at 6e-8 and takes the E3z line throughout.
+inline double tau_low_kh(int N, double s, bool fp64) { return fp64 ? s * (N < 64 ? 0.25 * N : 16.0) : -1.0; }
 
 __host__ __device__ inline int npar(int N, int g) { return (N + 1 - g) / 2; }  // #k in [0,N) with k%2 == g
 
@@ -72,8 +82,8 @@ inline TauShape tau_shape(int N, bool three) {
 // doubles per key of the set-up table: rows a_j of b, u, p (1 at k = 0, 1), responses p_1, u~_1, uz_1,
 // then scalars; after the last key the four coefficient rows of tau_coeffs
 enum { kTabB = 0, kTabU = 1, kTabP = 2, kTabP1 = 3, kTabX1 = 4, kTabZ1 = 5 };
-// scalars, [parity]: 1/sum of the homogeneous b, u, p lines; 1/q_1, tau_u1z of uz_1, top psi of u~_1 (by p's parity)
-// and alpha/beta, 1/alpha, beta, 1/beta of the b, u, p lines (kScLine + 4 op)
+// scalars, [parity]: 1/sum of the homogeneous b, u, p lines; 1/q_1 (q: the condition on lambda), tau_u1z of uz_1,
+// top psi of u~_1 (by p's parity) and alpha/beta, 1/alpha, beta, 1/beta of the b, u, p lines (kScLine + 4 op)
 enum { kScB = 0, kScU = 2, kScP = 4, kScQ = 6, kScTz = 8, kScPsi = 10, kScLine = 12 };
 constexpr int kTauScalars = 24;
 __host__ __device__ inline size_t tau_table_stride(const TauShape& h) { return (size_t)6 * tau_row(h) + kTauScalars; }
@@ -83,9 +93,9 @@ struct TauLine {
     double m, ial, beta, ibeta;  // alpha/beta, 1/alpha, beta, 1/beta
     bool psi;
 };
-__host__ __device__ inline TauLine tau_line(int N, double alpha, double beta) {
+__host__ __device__ inline TauLine tau_line(double alpha, double beta, double bound) {
     const double m = alpha / beta;
-    return TauLine{m, 1.0 / alpha, beta, 1.0 / beta, m > tau_psi_bound(N)};
+    return TauLine{m, 1.0 / alpha, beta, 1.0 / beta, m > bound};
 }
 // Row k of the second integral, relative to its r_{k-2} entry: t1 r_{k+2} - t2 r_k + g1 G_{k-1} - g2 G_{k+1},
 // with the lifts' changes in the top rows (A: rows N-3 and N-1, B: row N-2)
@@ -189,6 +199,7 @@ struct TauSys {
     const double* kh;        // |k_h| per key (null: kh = k0x * key)
     double k0x;
     double* table;           // tau_table_doubles
+    double bound, low;       // tau_psi_bound, tau_low_kh
 };
 __device__ inline double tau_kh(const TauSys& t, int key) { return t.kh ? t.kh[key] : t.k0x * key; }
 
@@ -205,9 +216,9 @@ static __global__ __launch_bounds__(64) void k_tau_setup(TauSys t) {
     for (int i = tid; i < 6 * N; i += 64) tab[i] = 0.0;
     if (tid < kTauScalars) sc[tid] = 0.0;
     __syncthreads();
-    const TauLine lb = tau_line(N, 1.0 + c * t.kappa * kh * kh, c * t.kappa * s * s);
-    const TauLine lu = tau_line(N, 1.0 + c * t.nu * kh * kh, c * t.nu * s * s);
-    const TauLine lp = tau_line(N, c * kh * kh, c * s * s);  // kh = 0: no line is solved with it (1/alpha is inf)
+    const TauLine lb = tau_line(1.0 + c * t.kappa * kh * kh, c * t.kappa * s * s, t.bound);
+    const TauLine lu = tau_line(1.0 + c * t.nu * kh * kh, c * t.nu * s * s, t.bound);
+    const TauLine lp = tau_line(c * kh * kh, c * s * s, t.bound);  // kh = 0: no line is solved with it (1/alpha is inf)
     if (tid < 3) {
         const TauLine L = tid == 0 ? lb : (tid == 1 ? lu : lp);
         double* o = sc + kScLine + 4 * tid;
@@ -223,6 +234,7 @@ static __global__ __launch_bounds__(64) void k_tau_setup(TauSys t) {
         const auto none = [](int) { return 0.0; };
         if (tid < 2) tau_solve_line(N, tid, lp, tab + kTabP * N, sc[kScP + tid], none, none, E, p1, 1.0);
         __syncthreads();
+        double q1 = 1.0;
         if (tid < 2) {
             const TauSums q = tau_solve_line(N, tid, lu, tab + kTabU * N, sc[kScU + tid],
                                              [&](int k) { return -c * kh * p1[k]; }, none, E + 2 * N, x1, 0.0);
@@ -232,9 +244,26 @@ static __global__ __launch_bounds__(64) void k_tau_setup(TauSys t) {
             const TauSums q = tau_solve_line(N, h, lu, tab + kTabU * N, sc[kScU + h], none,
                                              [&](int k) { return -c * s * p1[k]; }, E + 3 * N, z1, 0.0);
             const double tz = g == PL ? q.psi * s / (2.0 * (N - 1)) + p1[N - 1] * c * s * s * lu.ibeta : 0.0;
-            sc[kScQ + g] = 1.0 / (s * q.k2 + tz);
+            q1 = s * q.k2 + tz;
             sc[kScTz + g] = tz;
         }
+        __syncthreads();
+        if (kh <= t.low && tid >= 2 && tid < 4) {  // uz_1 as the integral of kh u~_1
+            const int h = tid - 2, g = h ^ 1;
+            double sum = 0.0;
+            for (int k = N - 1 - ((N - 1 - h) & 1); k >= 1; k -= 2) {
+                const double z = kh * ((k == 1 ? 2.0 : 1.0) * x1[k - 1] - (k + 1 <= N - 2 ? x1[k + 1] : 0.0)) / (2.0 * k * s);
+                z1[k] = z;
+                sum += z;
+            }
+            q1 = sum;
+            if (h == 0) {
+                q1 += z1[0];
+                z1[0] = -sum;
+            }
+            sc[kScTz + g] = g == PL ? kh * x1[N - 1] : 0.0;
+        }
+        if (tid >= 2 && tid < 4) sc[kScQ + ((tid - 2) ^ 1)] = 1.0 / q1;
         __syncthreads();
     }
     const int S = tau_row(t.shape);
@@ -445,6 +474,7 @@ template <typename T, bool THREE, int G, int E, bool PSI, bool HASD, bool MEAN>
 __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const TauArgs<T>& s, int slot0, int g, unsigned char* lds) {
 #pragma clang fp contract(off)
     using V = cplx<T>;
+    constexpr bool LOW = sizeof(T) == 8;  // tau_low_kh
     constexpr int NM = 64 / G, K = 2 * E, LS = (K + 1) * G;  // LDS: K + 1 values per lane, so lanes differ in bank
     const int lane = (int)threadIdx.x & 63, l = lane & (G - 1), grp = lane / G;
     const int N = s.t.N, S = K * G, k0 = K * l + g;  // own degrees: k0 + 2 i
@@ -545,7 +575,7 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
     auto coeff = [&](int r, int i) { return AHEAD ? cof[AHEAD ? r : 0][i] : co[r * S + 2 * i * G]; };
     auto line_of = [&](int op) {
         const double* q = sc + kScLine + 4 * op;
-        return TauLine{q[0], q[1], q[2], q[3], q[0] > tau_psi_bound(N)};
+        return TauLine{q[0], q[1], q[2], q[3], q[0] > s.t.bound};
     };
     // ---- right-hand sides ----
     Row b, x, z;
@@ -700,6 +730,13 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
         for (int i = 0; i < E; ++i) o = k0 + 2 * i == kt ? v[i][p] : o;
         return o;
     };
+    auto at_top_d = [&](int p) __attribute__((always_inline)) {
+        double o = 0.0;
+        if constexpr (HASD)
+#pragma unroll
+            for (int i = 0; i < E; ++i) o = k0 + 2 * i == kt ? d[i][p] : o;
+        return o;
+    };
     const double zero2[2] = {0.0, 0.0};
     const Nbr none{};
     double2* const park = reinterpret_cast<double2*>(lds + tau_pair_bytes<G, E>()) + 64 * E * g + lane;  // 3-D only
@@ -801,6 +838,7 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
         }
     }
     const bool mean = MEAN && kh == 0.0;
+    const bool low = LOW && kh <= s.t.low;  // uz from E1
     // ---- pressure, zero wall value of p - nu d ----
     Row q;
     double wd[2] = {0.0, 0.0};
@@ -832,7 +870,7 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
             }
     }
     // ---- u~, uz ----
-    double topx[2], topz[2], k2[2] = {0.0, 0.0};
+    double topx[2], topz[2], k2[2] = {0.0, 0.0}, zi[2] = {0.0, 0.0};
     {
         double a[E];
         table(kTabU, a);
@@ -853,8 +891,38 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
             for (int i = 0; i < E; ++i) {
                 const double k = k0 + 2 * i;
                 k2[p] = fma(k * k, z[i][p], k2[p]);
-                if constexpr (MEAN) z[i][p] = mean ? zm[i][p] : z[i][p];
+                if constexpr (MEAN && !LOW) z[i][p] = mean ? zm[i][p] : z[i][p];
             }
+        if constexpr (LOW) {
+            Row f;
+#pragma unroll
+            for (int i = 0; i < E; ++i)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+                    f[i][p] = k0 + 2 * i >= N - 1 ? 0.0 : fma(kh, x[i][p], HASD ? d[HASD ? i : 0][p] : 0.0);
+            swap(f, n);
+            double iz[E];
+#pragma unroll
+            for (int i = 0; i < E; ++i) iz[i] = 0.5 / (sz * (k0 + 2 * i > 0 ? k0 + 2 * i : 1));
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                double v[E], sum = 0.0;
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const int k = k0 + 2 * i;
+                    v[i] = k >= 1 && k < N ? ((k == 1 ? 2.0 : 1.0) * n[i][p] - n[i + 1][p]) * iz[i] : 0.0;
+                    sum += v[i];
+                }
+                sum = lanes_sum<G>(sum);
+                zi[p] = sum + lanes_sum<G>(k0 == 0 ? z[0][p] : 0.0);  // even: against the degree 0 of the line
+                if (k0 == 0) v[0] = -sum;
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    z[i][p] = low ? v[i] : z[i][p];
+                    if constexpr (MEAN) z[i][p] = mean ? zm[i][p] : z[i][p];
+                }
+            }
+        }
     }
     // ---- lambda per parity of p: E1 on the wall; uz has the other parity ----
     double lam[2], lamz[2], tz[2];  // lam: own parity; lamz: the other; tz: tau_u1z before the response
@@ -864,7 +932,7 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
             const double t = lanes_sum<G>(l == lt ? (A ? at_top(q, p) * (c * sz * sz * lu.ibeta) : topz[p] * tscale) : 0.0);
             k2[p] = lanes_sum<G>(k2[p]);
             if (l == 0) {
-                xs[8 * g + p] = k2[p];
+                xs[8 * g + p] = LOW && low ? zi[p] : k2[p];
                 xs[8 * g + 2 + p] = wd[p];
                 xs[8 * g + 4 + p] = t;
                 if constexpr (MEAN) xs[8 * g + 6 + p] = first[p];
@@ -875,8 +943,16 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             tz[p] = xs[4 + p] + xs[12 + p];
-            const double own = sz * xs[8 * (g ^ 1) + p] + (A ? tz[p] : 0.0) - xs[8 * g + 2 + p];
-            const double oth = sz * xs[8 * g + p] + (A ? 0.0 : tz[p]) - xs[8 * (g ^ 1) + 2 + p];
+            double own = sz * xs[8 * (g ^ 1) + p] + (A ? tz[p] : 0.0) - xs[8 * g + 2 + p];
+            double oth = sz * xs[8 * g + p] + (A ? 0.0 : tz[p]) - xs[8 * (g ^ 1) + 2 + p];
+            if (LOW) {
+                own = low ? xs[8 * (g ^ 1) + p] : own;
+                oth = low ? xs[8 * g + p] : oth;
+                if (A) {  // row N - 1 of E1
+                    const double t = fma(kh, at_top(x, p), HASD ? at_top_d(p) : 0.0);
+                    tz[p] = low ? t : tz[p];
+                }
+            }
             lam[p] = mean ? 0.0 : -own * iq;
             lamz[p] = mean ? 0.0 : -oth * iqz;
             if constexpr (MEAN) taup[p] -= sz * xs[8 + 6 + p];
@@ -1008,10 +1084,10 @@ inline void tau_flags(bool psi, bool hasd, F&& f) {
 }
 
 // whether any key up to kh_max takes the psi-form
-inline bool tau_uses_psi(int N, double c, double s, double kappa, double nu, double kh_max) {
-    const double lim = tau_psi_bound(N), k2 = kh_max * kh_max / (s * s);
-    const double mb = 1.0 / (c * kappa * s * s) + k2, mu = 1.0 / (c * nu * s * s) + k2;
-    return mb > lim || mu > lim;  // the pressure's m = k2 is below both
+inline bool tau_uses_psi(const TauSys& t, double kh_max) {
+    const double k2 = kh_max * kh_max / (t.s * t.s);  // m of the pressure lines, below those of b and u
+    const double mb = 1.0 / (t.c * t.kappa * t.s * t.s) + k2, mu = 1.0 / (t.c * t.nu * t.s * t.s) + k2;
+    return mb > t.bound || mu > t.bound;
 }
 
 }  // namespace tarang

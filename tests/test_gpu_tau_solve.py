@@ -13,6 +13,8 @@ is what an equation row leaves over, whose terms reach (1/dt + nu (2/Lz)^2 N^4) 
 import numpy as np
 import pytest
 
+from tarang_amd._lib import CHAN3_B, CHAN3_P, CHAN3_UX, CHAN3_UY, CHAN3_UZ, CHAN_B, CHAN_P, CHAN_UX, CHAN_UZ
+from tests.tau_reference import Mode
 from tests.test_gpu_channel import random_state
 from tests.test_gpu_channel3d import random_state3
 
@@ -69,3 +71,93 @@ def test_tau_solve_3d(gpu, oracle, N, form, ts):
     fields = (oracle.RBC3_B, oracle.RBC3_UX, oracle.RBC3_UY, oracle.RBC3_UZ)
     check(s, ref, fields, oracle.RBC3_P, 9, N, nu, dt)
     s.close()
+
+
+SCALE = 2.0 ** -600  # products of two state values underflow to zero: a step is its linear solve alone
+
+
+def spectrum(rng, shape, N):
+    """Random complex coefficients, falling off as a resolved field's do."""
+    return (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) * np.exp(-np.arange(N) * 30.0 / N)
+
+
+def parts(c):
+    return np.stack([c.real, c.imag], axis=-1)
+
+
+def check_precision(err, lu, what):
+    """Geometric means over the modes: within four times a dense FP64 elimination of the same systems (the
+    means of the two differ by up to 3.5 over the sizes here) plus a floor of 8 eps for small N."""
+    for f in err:
+        a, b = (float(np.exp(np.mean(np.log(np.maximum(v[f], 1e-18))))) for v in (err, lu))
+        print(f"  {what} {f}: {a:.1e}, dense FP64 {b:.1e}", flush=True)
+        assert a <= 4.0 * b + 8 * 2.3e-16, (what, f, a, b)
+
+
+@pytest.mark.parametrize("Lx", [40.0, 1.0])  # kh from 0.08 to 0.6 s, from 3 to 22 s: uz from E1, and both sides of the change
+@pytest.mark.parametrize("mr", [0.05, 1.0, 30.0, 1000.0])  # alpha/beta of the velocity lines over N^2
+@pytest.mark.parametrize("N", [16, 33, 97, 128])
+def test_tau_solve_precision_2d(gpu, N, mr, Lx):
+    """A linear FP64 step against long double: no further off than a dense FP64 elimination."""
+    print(f"tau solve precision 2-D N={N} m/N2={mr} Lx={Lx}", flush=True)
+    nx, Lz, dt = 16, 1.0, 2.0 ** -10  # a power of two: the right-hand side is the state itself
+    nu = 1.0 / (mr * N * N * dt * 4.0)
+    rng = np.random.default_rng(N)
+    st = {v: spectrum(rng, (nx // 2 + 1, N), N) for v in (CHAN_B, CHAN_UX, CHAN_UZ)}
+    for c in st.values():
+        c[[0, -1]] = c[[0, -1]].real
+    s = gpu.chan(nx, N, Lx, Lz, nu, nu, dt, stepper=4, b_bottom=0.0, b_top=0.0)
+    for v, c in st.items():
+        s.set(v, c * SCALE)
+    s.step(1)
+    got = {f: s.get(v) / SCALE for f, v in (("b", CHAN_B), ("u", CHAN_UX), ("uz", CHAN_UZ), ("p", CHAN_P))}
+    s.close()
+    err, lu = ({f: [] for f in got} for _ in range(2))
+    for m in range(nx // 2):
+        rhs = [parts(st[CHAN_B][m]), parts(-1j * st[CHAN_UX][m]), parts(st[CHAN_UZ][m])]
+        args = (N, 2 * np.pi * m / Lx, dt, nu, nu, 2.0 / Lz)
+        ref, dense = Mode(*args)(*rhs), Mode(*args, dtype=np.float64)(*rhs)
+        for f in got:
+            size = np.linalg.norm(ref[f].astype(float))
+            if m == 0 and f == "uz":
+                assert np.abs(got[f][0]).max() == 0.0  # E1 at kh = 0
+                continue
+            g = parts(-1j * got[f][m] if f == "u" else got[f][m])
+            err[f].append(float(np.linalg.norm((g - ref[f]).astype(float)) / size))
+            lu[f].append(float(np.linalg.norm((dense[f] - ref[f]).astype(float)) / size))
+    check_precision(err, lu, "2-D")
+
+
+@pytest.mark.parametrize("N,mr", [(33, 1000.0), (64, 30.0), (97, 1.0), (128, 30.0)])
+def test_tau_solve_precision_3d(gpu, N, mr):
+    print(f"tau solve precision 3-D N={N} m/N2={mr}", flush=True)
+    nx, ny, Lx, Ly, Lz, dt = 8, 8, 40.0, 1.5, 1.0, 2.0 ** -10
+    nu = 1.0 / (mr * N * N * dt * 4.0)
+    rng = np.random.default_rng(N)
+    fields = (CHAN3_B, CHAN3_UX, CHAN3_UY, CHAN3_UZ)
+    st = {v: spectrum(rng, (nx // 2 + 1, ny, N), N) for v in fields}
+    s = gpu.chan3(nx, ny, N, Lx, Ly, Lz, nu, nu, dt, stepper=4, b_bottom=0.0, b_top=0.0)
+    for v, c in st.items():
+        s.set(v, c * SCALE)
+    s.step(1)
+    o = {v: s.get(v) / SCALE for v in fields + (CHAN3_P,)}
+    s.close()
+    err, lu = ({f: [] for f in ("b", "u", "v", "uz", "p")} for _ in range(2))
+    for m in range(1, nx // 2):  # the kx = 0 and kx = Nx/2 lines are projected onto real fields
+        for n in list(range(ny // 2)) + list(range(ny // 2 + 1, ny)):
+            kx, ky = 2 * np.pi * m / Lx, 2 * np.pi * (n if n < ny // 2 else n - ny) / Ly
+            kh = np.hypot(kx, ky)
+            turn = lambda x, y: (parts(-1j * (kx * x + ky * y) / kh), parts(-1j * (-ky * x + kx * y) / kh))  # noqa: E731
+            rx, ry = turn(st[CHAN3_UX][m, n], st[CHAN3_UY][m, n])
+            rhs = [parts(st[CHAN3_B][m, n]), rx, parts(st[CHAN3_UZ][m, n]), ry]
+            args = (N, kh, dt, nu, nu, 2.0 / Lz)
+            if len(err["b"]) and n % 2:  # every other mode: the reference is slow
+                continue
+            ref, dense = Mode(*args)(*rhs), Mode(*args, dtype=np.float64)(*rhs)
+            u, v = turn(o[CHAN3_UX][m, n], o[CHAN3_UY][m, n])
+            got = {"b": parts(o[CHAN3_B][m, n]), "u": u, "v": v, "uz": parts(o[CHAN3_UZ][m, n]), "p": parts(o[CHAN3_P][m, n])}
+            for f in got:
+                size = np.linalg.norm(ref[f].astype(float))
+                err[f].append(float(np.linalg.norm((got[f] - ref[f]).astype(float)) / size))
+                lu[f].append(float(np.linalg.norm((dense[f] - ref[f]).astype(float)) / size))
+    check_precision(err, lu, "3-D")
