@@ -316,10 +316,10 @@ double Channel3Solver::implicit_c(bool first) const {
     return (1.0 + w) * d_.dt / (1.0 + 2.0 * w);
 }
 
-TauSys Channel3Solver::tau_sys() const {
+TauSys Channel3Solver::tau_sys(double c) const {
     const bool fp64 = d_.dtype == kF64;
     const double sz = 2.0 / d_.Lz;
-    return TauSys{d_.nz, tau_shape(d_.nz, true), nkeys_, factored_c_, sz, d_.kappa, d_.nu, kh_.as<const double>(), 0.0,
+    return TauSys{d_.nz, tau_shape(d_.nz, true), nkeys_, c, sz, d_.kappa, d_.nu, kh_.as<const double>(), 0.0,
                   tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
 }
 
@@ -334,11 +334,12 @@ void Channel3Solver::factor(double c) {
         if (d_.nu == 0.0) bad += " perp-system" + key + " u-p-system" + key;
     }
     TG_REQUIRE(bad.empty(), kErrSingular, "3-D channel solver: singular per-mode system:" + bad);
-    factored_c_ = c;
-    hipLaunchKernelGGL(k_tau_setup, dim3(nkeys_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream,
-                       tau_sys());
-    TG_HIP(hipGetLastError());
     invalidate_graph();
+    factored_c_ = -1;  // until the set-up is in the stream: a failed launch is not taken for done by the next step
+    hipLaunchKernelGGL(k_tau_setup, dim3(nkeys_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream,
+                       tau_sys(c));
+    TG_HIP(hipGetLastError());
+    factored_c_ = c;
 }
 
 template <typename T>
@@ -454,7 +455,7 @@ template <typename T>
 void Channel3Solver::solve_t() {
     using V = cplx<T>;
     TauArgs<T> a{};
-    a.t = tau_sys();
+    a.t = tau_sys(factored_c_);
     a.nmodes = nmodes_;
     a.bcv = bcv_.as<const double2>();
     a.modes = modes_.as<const int2>();

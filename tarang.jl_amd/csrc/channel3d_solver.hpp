@@ -81,7 +81,7 @@ class Channel3Solver {
     template <typename T> void transpose_t(const void* in, void* out, int rows, int cols);
     double implicit_c(bool first) const;
     bool first_step() const { return multistep() && (iter_ == 0 || d_.stepper == kSBDF1); }
-    TauSys tau_sys() const;
+    TauSys tau_sys(double c) const;
     void factor(double c);
     void autotune();
     void launch_step_body();

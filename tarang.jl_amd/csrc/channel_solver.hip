@@ -216,11 +216,11 @@ void ChannelSolver::factor(double c) {
         if (d_.nu == 0.0) bad += " u-p-system" + mode;
     }
     TG_REQUIRE(bad.empty(), kErrSingular, "channel solver: singular per-mode system:" + bad);
-    factored_c_ = c;
-    hipLaunchKernelGGL(k_tau_setup, dim3(nxh_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream,
-                       solve_args<double>().t);
-    TG_HIP(hipGetLastError());
     invalidate_graph();
+    factored_c_ = -1;  // until the set-up is in the stream: a failed launch is not taken for done by the next step
+    hipLaunchKernelGGL(k_tau_setup, dim3(nxh_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream, tau_sys(c));
+    TG_HIP(hipGetLastError());
+    factored_c_ = c;
 }
 
 // ---- kernels of one step ----
@@ -324,17 +324,21 @@ void ChannelSolver::stage_rhs_t(int st, bool final_update) {
     TG_HIP(hipGetLastError());
 }
 
+TauSys ChannelSolver::tau_sys(double c) const {
+    const bool fp64 = d_.dtype == kF64;
+    const double sz = 2.0 / d_.Lz;
+    return TauSys{d_.nz, tau_shape(d_.nz, false), nxh_, c, sz, d_.kappa, d_.nu, nullptr, 2.0 * M_PI / d_.Lx,
+                  tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
+}
+
 template <typename T>
 TauArgs<T> ChannelSolver::solve_args() const {
     using V = cplx<T>;
     TauArgs<T> a{};
-    const double k0x = 2.0 * M_PI / d_.Lx, sz = 2.0 / d_.Lz;
-    const bool fp64 = d_.dtype == kF64;
-    a.t = TauSys{d_.nz, tau_shape(d_.nz, false), nxh_, factored_c_, sz, d_.kappa, d_.nu, nullptr, k0x,
-                 tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
+    a.t = tau_sys(factored_c_);
     a.nmodes = nxh_;
     a.bcv = bcv_.as<const double2>();
-    a.psi = tau_uses_psi(a.t, k0x * (nxh_ - 1));
+    a.psi = tau_uses_psi(a.t, a.t.k0x * (nxh_ - 1));
     a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
     a.R2 = R_[1].as<const V>();
     a.R3x = R_[2].as<const V>();

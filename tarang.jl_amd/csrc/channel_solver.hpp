@@ -27,6 +27,7 @@ struct ChannelDesc {
 
 enum ChannelVar : int { kChP = 0, kChB = 1, kChUX = 2, kChUZ = 3 };
 
+struct TauSys;
 template <typename T> struct TauArgs;
 class ChannelGroup;
 
@@ -69,6 +70,7 @@ class ChannelSolver {
     int nsolves() const { return multistep() ? 1 : tab_.stages - 1; }
     void segment(int i);
     template <typename T> void segment_t(int i);
+    TauSys tau_sys(double c) const;
     template <typename T> TauArgs<T> solve_args() const;
     int solve_wgs() const;  // workgroups (waves) of the solve kernel
     void advance_clock();
