@@ -252,7 +252,8 @@ typedef struct {
 #define TARANG_CHAN_UX 2
 #define TARANG_CHAN_UZ 3
 
-/* builds and factors the per-mode systems for dt; TARANG_ERR_SINGULAR names singular modes */
+/* builds and factors the per-mode systems for dt; TARANG_ERR_SINGULAR names singular modes (a zero kappa or
+ * nu among them; negative ones are solved, with pivoting) */
 int tarang_chan_create(tarang_ctx_t ctx, const tarang_chan_desc* desc, tarang_chan_t* out);
 int tarang_chan_destroy(tarang_chan_t s);
 /* coefficient array of p, b, ux or uz: complex (nx/2+1, nz), reference layout, device pointer

@@ -148,7 +148,8 @@ Channel3Solver::Channel3Solver(Context* ctx, const Channel3Desc& d) : ctx_(ctx),
     up(kh_, khv.data(), khv.size() * sizeof(double));
     up(modes_, modes.data(), modes.size() * sizeof(int2));
     up(rot_, rot.data(), rot.size() * sizeof(double));
-    tab_tau_ = DevBuf(ctx_, tau_table_doubles(tau_shape(d.nz, true), nkeys_) * sizeof(double));
+    tab_tau_ = DevBuf(ctx_, tau_table_doubles(tau_shape(d.nz, true, any_sign()), nkeys_) * sizeof(double));
+    if (any_sign()) info_ = DevBuf(ctx_, nkeys_ * sizeof(int));
     {
         const auto bcv = constant_wall_values((size_t)nmodes_, (double)d.nx * d.ny, d.b_bottom, d.b_top);
         bcv_ = DevBuf(ctx_, bcv.size() * sizeof(double2));
@@ -319,26 +320,43 @@ double Channel3Solver::implicit_c(bool first) const {
 TauSys Channel3Solver::tau_sys(double c) const {
     const bool fp64 = d_.dtype == kF64;
     const double sz = 2.0 / d_.Lz;
-    return TauSys{d_.nz, tau_shape(d_.nz, true), nkeys_, c, sz, d_.kappa, d_.nu, kh_.as<const double>(), 0.0,
-                  tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
+    return TauSys{d_.nz, tau_shape(d_.nz, true, any_sign()), nkeys_, c, sz, d_.kappa, d_.nu, kh_.as<const double>(), 0.0,
+                  tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64), info_.as<int>()};
 }
+
+bool Channel3Solver::any_sign() const { return tau_any_sign(d_.kappa, d_.nu); }
 
 void Channel3Solver::factor(double c) {
     if (c == factored_c_) return;
-    // a vanishing diffusivity leaves the D T_{N-1} lift of its equation without a coefficient
+    const TauSys t = tau_sys(c);
     std::string bad;
-    const std::string par = ", parity " + std::to_string((d_.nz & 1) ? 1 : 0) + ")";  // parity of N - 2
+    const std::string par = ", parity " + std::to_string(d_.nz & 1) + ")";  // the parity of N - 2
     for (int k = 0; k < nkeys_ && bad.size() < 200; ++k) {
         const std::string key = "(|k_h| key " + std::to_string(k) + par;
-        if (d_.kappa == 0.0) bad += " b-system" + key;
-        if (d_.nu == 0.0) bad += " perp-system" + key + " u-p-system" + key;
+        if (tau_no_diffusion(c, t.s, d_.kappa)) bad += " b-system" + key;
+        if (tau_no_diffusion(c, t.s, d_.nu)) bad += " perp-system" + key + " u-p-system" + key;
     }
     TG_REQUIRE(bad.empty(), kErrSingular, "3-D channel solver: singular per-mode system:" + bad);
     invalidate_graph();
     factored_c_ = -1;  // until the set-up is in the stream: a failed launch is not taken for done by the next step
-    hipLaunchKernelGGL(k_tau_setup, dim3(nkeys_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream,
-                       tau_sys(c));
-    TG_HIP(hipGetLastError());
+    const size_t lds = tau_setup_lds(d_.nz, any_sign());
+    if (any_sign()) {
+        hipLaunchKernelGGL((k_tau_setup<true>), dim3(nkeys_), dim3(64), lds, ctx_->stream, t);
+        TG_HIP(hipGetLastError());
+        std::vector<int> info(nkeys_);
+        TG_HIP(hipMemcpyAsync(info.data(), info_.ptr, info.size() * sizeof(int), hipMemcpyDeviceToHost, ctx_->stream));
+        TG_HIP(hipStreamSynchronize(ctx_->stream));
+        for (int k = 0; k < nkeys_ && bad.size() < 200; ++k) {
+            const std::string key = "(|k_h| key " + std::to_string(k) + ")";
+            if (info[k] & 1) bad += " b-system" + key;
+            if (info[k] & 2) bad += " perp-system" + key;
+            if (info[k] & 6) bad += " u-p-system" + key;
+        }
+        TG_REQUIRE(bad.empty(), kErrSingular, "3-D channel solver: singular per-mode system:" + bad);
+    } else {
+        hipLaunchKernelGGL((k_tau_setup<false>), dim3(nkeys_), dim3(64), lds, ctx_->stream, t);
+        TG_HIP(hipGetLastError());
+    }
     factored_c_ = c;
 }
 
@@ -460,7 +478,7 @@ void Channel3Solver::solve_t() {
     a.bcv = bcv_.as<const double2>();
     a.modes = modes_.as<const int2>();
     a.rot = rot_.as<const double>();
-    a.psi = tau_uses_psi(a.t, kh_max_);
+    a.form = tau_form(a.t, kh_max_);
     a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
     a.R2 = R_[1].as<const V>();
     a.R3x = R_[2].as<const V>();
@@ -477,15 +495,21 @@ void Channel3Solver::solve_t() {
         constexpr int G = decltype(GC)::value, E = decltype(EC)::value;
         const unsigned np = tune_.solve == 1 ? 2 : 1, per = np * 64 / G;  // pairs of waves per workgroup
         const dim3 grid((nmodes_ + per - 1) / per), block(128 * np);
-        const size_t lds = np * (tau_pair_bytes<G, E>() + tau_park_bytes<G, E>());
-        auto go = [&](auto psi, auto hasd) {
-            hipLaunchKernelGGL((k3_tau_solve<T, G, E, decltype(psi)::value, decltype(hasd)::value>), grid, block, lds,
-                               ctx_->stream, a);
+        auto go = [&](auto form, auto hasd) {
+            constexpr int F = decltype(form)::value;
+            const size_t lds = np * tau_lds_bytes<G, E, true, F>();
+            hipLaunchKernelGGL((k3_tau_solve<T, G, E, F, decltype(hasd)::value>), grid, block, lds, ctx_->stream, a);
         };
-        tau_flags(a.psi, a.R1 != nullptr, go);
+        tau_flags(a.form, a.R1 != nullptr, go);
     };
     timed(6, [&] {
-        if (h.G == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 4>{});
+        if (a.form == kTauAny) {  // one mode per workgroup
+            constexpr size_t lds = tau_lds_bytes<64, 2, true, kTauAny>();
+            if (a.R1)
+                hipLaunchKernelGGL((k3_tau_solve<T, 64, 2, kTauAny, true>), dim3(nmodes_), dim3(128), lds, ctx_->stream, a);
+            else
+                hipLaunchKernelGGL((k3_tau_solve<T, 64, 2, kTauAny, false>), dim3(nmodes_), dim3(128), lds, ctx_->stream, a);
+        } else if (h.G == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 4>{});
         else if (h.E == 4) launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 4>{});
         else if (h.E == 2) launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 2>{});
         else launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
@@ -695,7 +719,8 @@ void Channel3Solver::kernel_bytes(double* out) const {
     out[4] = (8 * nc) * vb + N * N * rb;                        // read 4 planes, write 4 rows
     out[5] = (4 * 4 + 4 + 5) * nc * vb;                         // state (x2 on the kx lines), F, histories, rhs
     // solve: rhs rows and the per-key tables in, five fields out
-    out[6] = (multistep() ? 9 : 10) * nc * vb + (double)nkeys_ * tau_table_stride(tau_shape(d_.nz, true)) * sizeof(double);
+    out[6] = (multistep() ? 9 : 10) * nc * vb +
+             (double)nkeys_ * tau_table_stride(tau_shape(d_.nz, true, any_sign())) * sizeof(double);
     out[7] = 10 * nc * vb;  // L x: read p, b, u (and partners on two lines), write five rows
 }
 
@@ -717,7 +742,9 @@ size_t footprint(const Channel3Desc& d) {
     size_t b = nfields * alloc_granule(fb) + alloc_granule(kCh3ZPlanes * fb) + alloc_granule(kCh3Planes * prow) +
                alloc_granule(4 * prow);                                                           // G, Q, H
     b += alloc_granule(nmodes * kCh3TauStride * vb) + 3 * alloc_granule(N * N * ib);           // taus, tables
-    b += alloc_granule(tau_table_doubles(tau_shape(d.nz, true), keys) * sizeof(double));  // tau-solve tables
+    const bool any = tau_any_sign(d.kappa, d.nu);
+    b += alloc_granule(tau_table_doubles(tau_shape(d.nz, true, any), keys) * sizeof(double));  // tau-solve tables
+    if (any) b += alloc_granule(keys * sizeof(int));
     b += 8 * alloc_granule(nmodes * 32);                                 // keys, rotations, modes, walls
     return b;
 }

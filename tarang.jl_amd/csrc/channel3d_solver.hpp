@@ -82,6 +82,7 @@ class Channel3Solver {
     double implicit_c(bool first) const;
     bool first_step() const { return multistep() && (iter_ == 0 || d_.stepper == kSBDF1); }
     TauSys tau_sys(double c) const;
+    bool any_sign() const;  // a negative diffusivity
     void factor(double c);
     void autotune();
     void launch_step_body();
@@ -107,6 +108,7 @@ class Channel3Solver {
     DevBuf kh_, rot_, modes_;
     DevBuf bcv_, bch_;  // per-mode wall values of b [2 m + w], and the x-transform scratch
     DevBuf tab_tau_;  // per-key tables of the direct tau solves (tau_table_stride(nz) doubles each)
+    DevBuf info_;     // a negative diffusivity: zero pivots per key
     Chan3Tuning tune_;
     double kh_max_ = 0;
     bool graph_on_ = true;

@@ -100,7 +100,8 @@ ChannelSolver::ChannelSolver(Context* ctx, const ChannelDesc& d) : ctx_(ctx), d_
     upload(BT_, BT);
     upload(BDT_, BDT);
     upload(FT_, FT);
-    tab_tau_ = DevBuf(ctx_, tau_table_doubles(tau_shape(d.nz, false), nxh_) * sizeof(double));
+    tab_tau_ = DevBuf(ctx_, tau_table_doubles(tau_shape(d.nz, false, any_sign()), nxh_) * sizeof(double));
+    if (any_sign()) info_ = DevBuf(ctx_, nxh_ * sizeof(int));
     {
         const auto bcv = constant_wall_values((size_t)nxh_, (double)d.nx, d.b_bottom, d.b_top);
         bcv_ = DevBuf(ctx_, bcv.size() * sizeof(double2));
@@ -206,20 +207,34 @@ void ChannelSolver::set_dt(double dt) {
 // ---- implicit systems ----
 void ChannelSolver::factor(double c) {
     if (c == factored_c_) return;
-    // a vanishing diffusivity leaves the D T_{N-1} lift of its equation without a coefficient
+    const TauSys t = tau_sys(c);
     std::string bad;
-    const int gb = (d_.nz & 1) ? 1 : 0;  // parity of N - 2
-    const std::string par = ", parity " + std::to_string(gb) + ")";
+    const std::string par = ", parity " + std::to_string(d_.nz & 1) + ")";  // the parity of N - 2
     for (int m = 0; m < nxh_ && bad.size() < 200; ++m) {
         const std::string mode = "(kx mode " + std::to_string(m) + par;
-        if (d_.kappa == 0.0) bad += " b-system" + mode;
-        if (d_.nu == 0.0) bad += " u-p-system" + mode;
+        if (tau_no_diffusion(c, t.s, d_.kappa)) bad += " b-system" + mode;
+        if (tau_no_diffusion(c, t.s, d_.nu)) bad += " u-p-system" + mode;
     }
     TG_REQUIRE(bad.empty(), kErrSingular, "channel solver: singular per-mode system:" + bad);
     invalidate_graph();
     factored_c_ = -1;  // until the set-up is in the stream: a failed launch is not taken for done by the next step
-    hipLaunchKernelGGL(k_tau_setup, dim3(nxh_), dim3(64), (size_t)10 * d_.nz * sizeof(double), ctx_->stream, tau_sys(c));
-    TG_HIP(hipGetLastError());
+    const size_t lds = tau_setup_lds(d_.nz, any_sign());
+    if (any_sign()) {
+        hipLaunchKernelGGL((k_tau_setup<true>), dim3(nxh_), dim3(64), lds, ctx_->stream, t);
+        TG_HIP(hipGetLastError());
+        std::vector<int> info(nxh_);
+        TG_HIP(hipMemcpyAsync(info.data(), info_.ptr, info.size() * sizeof(int), hipMemcpyDeviceToHost, ctx_->stream));
+        TG_HIP(hipStreamSynchronize(ctx_->stream));
+        for (int m = 0; m < nxh_ && bad.size() < 200; ++m) {
+            const std::string mode = "(kx mode " + std::to_string(m) + ")";
+            if (info[m] & 1) bad += " b-system" + mode;
+            if (info[m] & 6) bad += " u-p-system" + mode;
+        }
+        TG_REQUIRE(bad.empty(), kErrSingular, "channel solver: singular per-mode system:" + bad);
+    } else {
+        hipLaunchKernelGGL((k_tau_setup<false>), dim3(nxh_), dim3(64), lds, ctx_->stream, t);
+        TG_HIP(hipGetLastError());
+    }
     factored_c_ = c;
 }
 
@@ -327,9 +342,11 @@ void ChannelSolver::stage_rhs_t(int st, bool final_update) {
 TauSys ChannelSolver::tau_sys(double c) const {
     const bool fp64 = d_.dtype == kF64;
     const double sz = 2.0 / d_.Lz;
-    return TauSys{d_.nz, tau_shape(d_.nz, false), nxh_, c, sz, d_.kappa, d_.nu, nullptr, 2.0 * M_PI / d_.Lx,
-                  tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64)};
+    return TauSys{d_.nz, tau_shape(d_.nz, false, any_sign()), nxh_, c, sz, d_.kappa, d_.nu, nullptr, 2.0 * M_PI / d_.Lx,
+                  tab_tau_.as<double>(), tau_psi_bound(d_.nz, fp64), tau_low_kh(d_.nz, sz, fp64), info_.as<int>()};
 }
+
+bool ChannelSolver::any_sign() const { return tau_any_sign(d_.kappa, d_.nu); }
 
 template <typename T>
 TauArgs<T> ChannelSolver::solve_args() const {
@@ -338,7 +355,7 @@ TauArgs<T> ChannelSolver::solve_args() const {
     a.t = tau_sys(factored_c_);
     a.nmodes = nxh_;
     a.bcv = bcv_.as<const double2>();
-    a.psi = tau_uses_psi(a.t, a.t.k0x * (nxh_ - 1));
+    a.form = tau_form(a.t, a.t.k0x * (nxh_ - 1));
     a.R1 = multistep() ? nullptr : R_[0].as<const V>();  // the multistep E1 rows are zero
     a.R2 = R_[1].as<const V>();
     a.R3x = R_[2].as<const V>();
@@ -352,7 +369,7 @@ TauArgs<T> ChannelSolver::solve_args() const {
 }
 
 int ChannelSolver::solve_wgs() const {
-    const int per = 64 / tau_shape(d_.nz, false).G;
+    const int per = 64 / tau_shape(d_.nz, false, any_sign()).G;
     return (nxh_ + per - 1) / per;
 }
 
@@ -363,14 +380,17 @@ void ChannelSolver::solve_t() {
     const unsigned nwg = (unsigned)solve_wgs();
     auto launch = [&](auto GC, auto EC) {
         constexpr int G = decltype(GC)::value, E = decltype(EC)::value;
-        auto go = [&](auto psi, auto hasd) {
-            hipLaunchKernelGGL((k_ch_tau_solve<T, G, E, decltype(psi)::value, decltype(hasd)::value>), dim3(nwg),
+        auto go = [&](auto form, auto hasd) {
+            hipLaunchKernelGGL((k_ch_tau_solve<T, G, E, decltype(form)::value, decltype(hasd)::value>), dim3(nwg),
                                dim3(128), 0, ctx_->stream, sa);
         };
-        tau_flags(sa.psi, sa.R1 != nullptr, go);
+        tau_flags(sa.form, sa.R1 != nullptr, go);
     };
     timed(4, [&] {
-        if (h.G == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 1>{});
+        if (sa.form == kTauAny) {
+            if (sa.R1) hipLaunchKernelGGL((k_ch_tau_solve<T, 64, 4, kTauAny, true>), dim3(nwg), dim3(128), 0, ctx_->stream, sa);
+            else hipLaunchKernelGGL((k_ch_tau_solve<T, 64, 4, kTauAny, false>), dim3(nwg), dim3(128), 0, ctx_->stream, sa);
+        } else if (h.G == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 1>{});
         else if (h.E == 1) launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 1>{});
         else if (h.E == 2) launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
         else launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
@@ -578,7 +598,7 @@ void ChannelSolver::kernel_bytes(double* out) const {
     out[2] = (3 * nc + 3 * nc) * vb + N * N * rb;       // read 3 planes, write 3 F
     out[3] = (4 * nc + 4 * nc) * vb;                    // read p, b, ux, uz; write 4 rows
     // solve: read the rhs rows and the per-mode table, write 4 fields
-    out[4] = (multistep() ? 7 : 8) * nc * vb + (double)nxh_ * tau_table_stride(tau_shape(d_.nz, false)) * sizeof(double);
+    out[4] = (multistep() ? 7 : 8) * nc * vb + (double)nxh_ * tau_table_stride(tau_shape(d_.nz, false, any_sign())) * sizeof(double);
     out[5] = 0;
 }
 
@@ -597,7 +617,9 @@ size_t footprint(const ChannelDesc& d) {
     const size_t ib = dtype_size((DType)d.dtype);
     size_t b = nfields * alloc_granule(fb) + alloc_granule(8 * fb) + alloc_granule(3 * fb);  // G, H
     b += alloc_granule(nxh * 8 * vb) + 3 * alloc_granule(N * N * ib);                       // taus, tables
-    b += alloc_granule(tau_table_doubles(tau_shape(d.nz, false), nxh) * sizeof(double));                    // tau-solve tables
+    const bool any = tau_any_sign(d.kappa, d.nu);
+    b += alloc_granule(tau_table_doubles(tau_shape(d.nz, false, any), nxh) * sizeof(double));  // tau-solve tables
+    if (any) b += alloc_granule(nxh * sizeof(int));
     b += 2 * alloc_granule(2 * nxh * sizeof(double2));                                       // walls
     return b;
 }
@@ -622,35 +644,38 @@ ChannelGroup::ChannelGroup(const std::vector<ChannelSolver*>& members) : m_(memb
                    kErrInvalid, "channel group: members must share dtype, timestepper, refine_sweeps and split_inverse");
     }
     ctx_ = m_[0]->ctx_;
-    for (ChannelSolver* s : m_) total_wg_ += s->solve_wgs();
+    for (ChannelSolver* s : m_) (s->any_sign() ? alone_ : joint_).push_back(s);
+    for (ChannelSolver* s : joint_) total_wg_ += s->solve_wgs();
 }
 
 ChannelGroup::~ChannelGroup() { invalidate_graph(); }
 
 template <typename T>
 void ChannelGroup::fill_items() {
-    std::vector<TauItem<T>> it(m_.size());
+    std::vector<TauItem<T>> it(joint_.size());
     int wg0 = 0;
-    for (size_t i = 0; i < m_.size(); ++i) {
-        ChannelSolver* s = m_[i];
+    for (size_t i = 0; i < joint_.size(); ++i) {
+        ChannelSolver* s = joint_[i];
         it[i].s = s->solve_args<T>();
         it[i].wg0 = wg0;
         wg0 += s->solve_wgs();
     }
-    int psi = 0;  // one kernel for the group: the psi-form variant when any member needs it
-    for (auto& i : it) psi |= i.s.psi;
-    for (auto& i : it) i.s.psi = psi;
+    int form = kTauU;  // one kernel for the group: the psi-form variant when any member needs it
+    for (auto& i : it) form = std::max(form, i.s.form);
+    for (auto& i : it) i.s.form = form;
     hitems_.resize(it.size() * sizeof(TauItem<T>));
     std::memcpy(hitems_.data(), it.data(), hitems_.size());
 }
 
 template <typename T>
 void ChannelGroup::solve_group_t() {
+    for (ChannelSolver* s : alone_) s->solve_t<T>();
+    if (joint_.empty()) return;
     const TauItem<T>* items = items_.as<const TauItem<T>>();
-    const int n = (int)m_.size();
+    const int n = (int)joint_.size();
     const TauArgs<T>& first = reinterpret_cast<const TauItem<T>*>(hitems_.data())->s;  // flags group-wide (fill_items)
-    tau_flags(first.psi, first.R1 != nullptr, [&](auto psi, auto hasd) {
-        hipLaunchKernelGGL((k_ch_tau_solve_group<T, decltype(psi)::value, decltype(hasd)::value>), dim3(total_wg_),
+    tau_flags(first.form, first.R1 != nullptr, [&](auto form, auto hasd) {
+        hipLaunchKernelGGL((k_ch_tau_solve_group<T, decltype(form)::value, decltype(hasd)::value>), dim3(total_wg_),
                            dim3(128), 0, ctx_->stream, items, n);
     });
     TG_HIP(hipGetLastError());
@@ -684,7 +709,8 @@ void ChannelGroup::step_once() {
         else fill_items<double>();
         if (items_.bytes < hitems_.size()) items_ = DevBuf(ctx_, hitems_.size());
         // stream-ordered after the previous step's launches, which read the old table
-        TG_HIP(hipMemcpyAsync(items_.ptr, hitems_.data(), hitems_.size(), hipMemcpyHostToDevice, ctx_->stream));
+        if (!hitems_.empty())
+            TG_HIP(hipMemcpyAsync(items_.ptr, hitems_.data(), hitems_.size(), hipMemcpyHostToDevice, ctx_->stream));
         TG_HIP(hipStreamSynchronize(ctx_->stream));
         graph_key_ = key;
     }

@@ -71,6 +71,7 @@ class ChannelSolver {
     void segment(int i);
     template <typename T> void segment_t(int i);
     TauSys tau_sys(double c) const;
+    bool any_sign() const;  // a negative diffusivity
     template <typename T> TauArgs<T> solve_args() const;
     int solve_wgs() const;  // workgroups (waves) of the solve kernel
     void advance_clock();
@@ -112,6 +113,7 @@ class ChannelSolver {
     DevBuf BT_, BDT_, FT_;
     DevBuf bcv_, bch_;  // per-mode wall values of b [2 m + w], and the x-transform scratch
     DevBuf tab_tau_;    // per-mode tables of the direct tau solves (tau_table_stride(nz) doubles each)
+    DevBuf info_;       // a negative diffusivity: zero pivots per mode
     bool graph_on_ = true;
     hipGraphExec_t graph_ = nullptr;
     double graph_dt_ = 0, graph_dtp_ = 0;
@@ -145,6 +147,7 @@ class ChannelGroup {
         graph_ = nullptr;
     }
     std::vector<ChannelSolver*> m_;
+    std::vector<ChannelSolver*> joint_, alone_;  // solved in one launch; each by its own (a negative diffusivity)
     Context* ctx_;
     DevBuf items_;
     std::vector<unsigned char> hitems_, uploaded_;  // item table built for this step / on the device

@@ -70,11 +70,17 @@ __host__ __device__ inline int npar(int N, int g) { return (N + 1 - g) / 2; }  /
 struct TauShape {
     int G, E;
 };
+// Which recursion the solves run: kTauU and kTauPsi eliminate without pivoting, which the M-matrix of positive
+// diffusivities allows; with a negative one (kTauAny) the lines of m <= 0 are solved by tau_bordered.
+enum TauForm : int { kTauU = 0, kTauPsi = 1, kTauAny = 2 };
+inline bool tau_any_sign(double kappa, double nu) { return kappa < 0.0 || nu < 0.0; }
 __host__ __device__ inline int tau_row(const TauShape& h) { return 2 * h.E * h.G; }
 __host__ __device__ inline int tau_slot(const TauShape& h, int k) { return (k % (2 * h.E)) * h.G + k / (2 * h.E); }
 // 3-D: four modes per pair of waves up to N = 128 (scans stay within the 16-lane rows of the DPP shifts),
 // two above; 2-D has few modes: as many lanes per mode as degrees allow
-inline TauShape tau_shape(int N, bool three) {
+// (any sign: one shape for all N, one mode per pair of waves)
+inline TauShape tau_shape(int N, bool three, bool any) {
+    if (any) return three ? TauShape{64, 2} : TauShape{64, 4};
     if (three) return N <= 32 ? TauShape{16, 1} : N <= 64 ? TauShape{16, 2} : N <= 128 ? TauShape{16, 4} : TauShape{32, 4};
     return N <= 64 ? TauShape{32, 1} : N <= 128 ? TauShape{64, 1} : N <= 256 ? TauShape{64, 2} : TauShape{64, 4};
 }
@@ -95,8 +101,10 @@ struct TauLine {
 };
 __host__ __device__ inline TauLine tau_line(double alpha, double beta, double bound) {
     const double m = alpha / beta;
-    return TauLine{m, 1.0 / alpha, beta, 1.0 / beta, m > bound};
+    return TauLine{m, 1.0 / alpha, beta, 1.0 / beta, fabs(m) > bound};
 }
+// the r_{k-2} entry of row k of the second integral, k >= 2
+__host__ __device__ inline double tau_lo(int k) { return (k == 2 ? 2.0 : 1.0) / (4.0 * k * (k - 1.0)); }
 // Row k of the second integral, relative to its r_{k-2} entry: t1 r_{k+2} - t2 r_k + g1 G_{k-1} - g2 G_{k+1},
 // with the lifts' changes in the top rows (A: rows N-3 and N-1, B: row N-2)
 struct TauCoeffs {
@@ -122,14 +130,14 @@ __host__ __device__ inline double tau_factor_line(int N, int g, double m, double
         W = 1.0 + a[N - 1];
     } else {
         const int k = N - 2;
-        const double lo = (k == 2 ? 2.0 : 1.0) / (4.0 * k * (k - 1)), cb = k == 2 ? 0.5 : 1.0;
+        const double lo = tau_lo(k), cb = k == 2 ? 0.5 : 1.0;
         an = m * lo / (1.0 + m * lo * cb);
         a[k] = an;
         W = 1.0 + an;
     }
     for (; j >= 1; --j) {
         const int k = 2 * j + g;
-        const double lo = (k == 2 ? 2.0 : 1.0) / (4.0 * k * (k - 1));
+        const double lo = tau_lo(k);
         const bool up = !(A && j == n - 2);
         const double den = 1.0 + m / (2.0 * ((double)k * k - 1.0)) - (up ? m / (4.0 * k * (k + 1)) * an : 0.0);
         an = m * lo / den;
@@ -139,18 +147,65 @@ __host__ __device__ inline double tau_factor_line(int N, int g, double m, double
     return 1.0 / W;
 }
 
+// One line by pivoted elimination, for m of any sign: the rows j = 1 .. n-1 of the recursion (in columns
+// j-1, j, j+1) are upper triangular when row j pivots column j-1, and the wall sum is a last row of ones.  Each
+// step eliminates with the larger of the band row and that last row, which stays constant beyond its two
+// leading entries, so a line costs O(n).  S: five doubles per row, S[5 j + 4] the right-hand side of row j on
+// entry and u_j on return; wt: the wall sum.  False: an exactly zero pivot (the line is singular).
+// Against long-double solves: 2e-15 of the line's 2-norm up to m = -10 N^2; beyond, where the 1 of a row is
+// small beside m/(4 k^2) and nothing resolves the solution, up to 1e-13 (m = -300 N^2).
+__host__ __device__ inline bool tau_bordered(int N, int g, double m, double wt, double* S) {
+    const int n = npar(N, g);
+    double d0 = 1.0, d1 = 1.0, dt = 1.0, dr = wt;  // the last row: columns j, j + 1, beyond; right-hand side
+    bool ok = true;
+    for (int j = 0; j < n - 1; ++j) {
+        const int k = 2 * (j + 1) + g;
+        const TauCoeffs t = tau_coeffs(N, k);
+        const double lo = m * tau_lo(k), b0 = -lo, b1 = 1.0 + lo * t.t2, b2 = -lo * t.t1, br = S[5 * (j + 1) + 4];
+        double* U = S + 5 * j;
+        if (fabs(b0) >= fabs(d0)) {
+            const double l = d0 / b0;
+            ok = ok && b0 != 0.0;
+            U[0] = b0, U[1] = b1, U[2] = b2, U[3] = 0.0, U[4] = br;
+            d0 = d1 - l * b1;
+            d1 = dt - l * b2;
+            dr -= l * br;
+        } else {
+            const double l = b0 / d0;
+            U[0] = d0, U[1] = d1, U[2] = dt, U[3] = dt, U[4] = dr;
+            d0 = b1 - l * d1;
+            d1 = b2 - l * dt;
+            dt = -l * dt;
+            dr = br - l * dr;
+        }
+    }
+    ok = ok && d0 != 0.0;
+    double x1 = dr / d0, x2 = 0.0, tail = 0.0;  // u_{j+1}, u_{j+2}, sum beyond
+    S[5 * (n - 1) + 4] = x1;
+    for (int j = n - 2; j >= 0; --j) {
+        double* U = S + 5 * j;
+        const double x = (U[4] - U[1] * x1 - U[2] * x2 - U[3] * tail) / U[0];
+        U[4] = x;
+        tail += x2;
+        x2 = x1;
+        x1 = x;
+    }
+    return ok;
+}
+
 struct TauSums {
     double k2;   // sum k^2 u_k
     double psi;  // B: psi at degree N - 2 (the D T_{N-1} amplitude before the G term)
+    bool ok = true;  // no zero pivot
 };
 
 // One line of parity g by one thread (set-up, and the reference of the wave-parallel solve): r(k), G(k)
-// read the data, e is scratch, iW = tau_factor_line's result.
-template <typename RF, typename GF>
+// read the data, e is scratch (ANY: 5 npar doubles, else N), iW = tau_factor_line's result.
+template <bool ANY, typename RF, typename GF>
 __host__ __device__ inline TauSums tau_solve_line(int N, int g, const TauLine& L, const double* a, double iW, RF r, GF G,
                                                   double* e, double* u, double w) {
     const int n = npar(N, g);
-    const bool A = g == ((N - 1) & 1);
+    const bool A = g == ((N - 1) & 1), piv = ANY && !(L.m > 0.0);
     auto rr = [&](int k) { return k >= N - 1 + (A ? 0 : 1) ? 0.0 : r(k); };  // r_{N-1} is the tau_*2 row
     auto GG = [&](int k) { return k >= N ? 0.0 : G(k); };
     double en = 0.0;
@@ -158,29 +213,40 @@ __host__ __device__ inline TauSums tau_solve_line(int N, int g, const TauLine& L
         const int k = 2 * j + g;
         const TauCoeffs t = tau_coeffs(N, k);
         const double dg = t.g1 * GG(k - 1) - t.g2 * GG(k + 1);
-        en = a[k] * (t.t1 * en - L.ial * (L.psi ? 2.0 * k * t.g1 * rr(k) + L.m * dg
-                                               : rr(k - 2) + t.t1 * rr(k + 2) - t.t2 * rr(k) + dg));
-        e[k] = en;
+        const double f = L.psi ? 2.0 * k * t.g1 * rr(k) + L.m * dg : rr(k - 2) + t.t1 * rr(k + 2) - t.t2 * rr(k) + dg;
+        if (piv) {
+            e[5 * j + 4] = -tau_lo(k) * L.ibeta * f;
+        } else {
+            en = a[k] * (t.t1 * en - L.ial * f);
+            e[k] = en;
+        }
     }
     double Q = 0.0, sum = 0.0, rs = rr(g);
     for (int j = 1; j < n; ++j) {
         const int k = 2 * j + g;
-        Q = a[k] * Q + e[k];
-        sum += Q;
+        if (!piv) {
+            Q = a[k] * Q + e[k];
+            sum += Q;
+        }
         rs += rr(k);
     }
-    double x = ((L.psi ? L.m * w - rs * L.ibeta : w) - sum) * iW, est = 0.0, su = 0.0, sa = 0.0;
+    const double wt = L.psi ? L.m * w - rs * L.ibeta : w, ft = piv ? fabs(e[5 * (n - 1) + 4]) : 0.0;
+    double x = 0.0, est = 0.0, su = 0.0, sa = 0.0;
     TauSums out{0.0, 0.0};
+    if (piv) out.ok = tau_bordered(N, g, L.m, wt, e);
+    else x = (wt - sum) * iW;
     for (int j = 0; j < n; ++j) {
         const int k = 2 * j + g;
-        if (j > 0) x = a[k] * x + e[k];
+        if (piv) x = e[5 * j + 4];
+        else if (j > 0) x = a[k] * x + e[k];
         double v = L.psi ? (L.beta * x + rr(k)) * L.ial : x;
         if (L.psi && A) {  // u_{N-1}: the wall sum's remainder where the recursion has lost more
             if (k < N - 1) {
-                est = (j > 0 ? a[k] * est : 0.0) + fabs(x);
+                est = (piv || j == 0 ? 0.0 : a[k] * est) + fabs(x);
                 su += v;
                 sa += fabs(v);
-            } else if ((a[k] * est + fabs(e[k])) * L.beta * L.ial > sa + fabs(w)) {
+            } else if ((piv ? fabs(L.m) * tau_lo(k) * est + ft : a[k] * est + fabs(e[k])) * fabs(L.beta * L.ial) >
+                       sa + fabs(w)) {
                 v = w - su;
             }
         }
@@ -200,49 +266,65 @@ struct TauSys {
     double k0x;
     double* table;           // tau_table_doubles
     double bound, low;       // tau_psi_bound, tau_low_kh
+    int* info;               // any sign: per key, the systems that met a zero pivot (bit 0 b, 1 perp, 2 u-p)
 };
 __device__ inline double tau_kh(const TauSys& t, int key) { return t.kh ? t.kh[key] : t.k0x * key; }
+// set-up LDS: 6 N doubles of table rows, and the scratch of the lines that run side by side
+inline size_t tau_setup_lds(int N, bool any) {
+    return (size_t)(6 * N + (any ? 2 * 5 * npar(N, 0) : 4 * N)) * sizeof(double);
+}
 
 // The set-up table of one key per workgroup (64 threads): six lanes run the factor recursions, then
-// the lambda = 1 responses run as lines of their own.  LDS: 10 N doubles.
-static __global__ __launch_bounds__(64) void k_tau_setup(TauSys t) {
+// the lambda = 1 responses run as lines of their own.  LDS: tau_setup_lds.
+template <bool ANY>
+__global__ __launch_bounds__(64) void k_tau_setup(TauSys t) {
     extern __shared__ unsigned char smem_raw[];
     const int N = t.N, key = (int)blockIdx.x, tid = (int)threadIdx.x;
     double* tab = reinterpret_cast<double*>(smem_raw);  // [6][N]
-    double* E = tab + 6 * N;                             // [4][N] scratch rows
+    double* E = tab + 6 * N + (ANY ? (tid & 1) * 5 * npar(N, 0) : (tid & 3) * N);  // scratch row of a thread at work
     __shared__ double sc[kTauScalars];
+    __shared__ int bad;
     const double kh = tau_kh(t, key), c = t.c, s = t.s;
     const int PL = (N - 1) & 1;
     for (int i = tid; i < 6 * N; i += 64) tab[i] = 0.0;
     if (tid < kTauScalars) sc[tid] = 0.0;
+    if (tid == 0) bad = 0;
     __syncthreads();
     const TauLine lb = tau_line(1.0 + c * t.kappa * kh * kh, c * t.kappa * s * s, t.bound);
     const TauLine lu = tau_line(1.0 + c * t.nu * kh * kh, c * t.nu * s * s, t.bound);
     const TauLine lp = tau_line(c * kh * kh, c * s * s, t.bound);  // kh = 0: no line is solved with it (1/alpha is inf)
+    const auto none = [](int) { return 0.0; };
     if (tid < 3) {
         const TauLine L = tid == 0 ? lb : (tid == 1 ? lu : lp);
         double* o = sc + kScLine + 4 * tid;
         o[0] = L.m, o[1] = kh > 0.0 || tid < 2 ? L.ial : 0.0, o[2] = L.beta, o[3] = L.ibeta;
     }
+    if (ANY)  // the pivots of the b and u lines, each in place of its factors
+        for (int op = 0; op < 2; ++op) {
+            const TauLine L = op == 0 ? lb : lu;
+            if (tid < 2 && !(L.m > 0.0) && !tau_bordered(N, tid, L.m, 0.0, E)) atomicOr(&bad, op == 0 ? 1 : 2);
+        }
     if (tid < 6) {
         const int op = tid >> 1, g = tid & 1;
-        sc[2 * op + g] = tau_factor_line(N, g, op == 0 ? lb.m : (op == 1 ? lu.m : lp.m), tab + op * N);
+        const double m = op == 0 ? lb.m : (op == 1 ? lu.m : lp.m);
+        if (!ANY || m > 0.0) sc[2 * op + g] = tau_factor_line(N, g, m, tab + op * N);
     }
     __syncthreads();
     if (kh > 0.0) {
         double *p1 = tab + kTabP1 * N, *x1 = tab + kTabX1 * N, *z1 = tab + kTabZ1 * N;
-        const auto none = [](int) { return 0.0; };
-        if (tid < 2) tau_solve_line(N, tid, lp, tab + kTabP * N, sc[kScP + tid], none, none, E, p1, 1.0);
+        if (tid < 2) tau_solve_line<ANY>(N, tid, lp, tab + kTabP * N, sc[kScP + tid], none, none, E, p1, 1.0);
         __syncthreads();
         double q1 = 1.0;
         if (tid < 2) {
-            const TauSums q = tau_solve_line(N, tid, lu, tab + kTabU * N, sc[kScU + tid],
-                                             [&](int k) { return -c * kh * p1[k]; }, none, E + 2 * N, x1, 0.0);
+            const TauSums q = tau_solve_line<ANY>(N, tid, lu, tab + kTabU * N, sc[kScU + tid],
+                                                  [&](int k) { return -c * kh * p1[k]; }, none, E, x1, 0.0);
             sc[kScPsi + tid] = q.psi;
-        } else if (tid < 4) {
+        }
+        if (ANY) __syncthreads();  // two scratch rows
+        if (tid >= 2 && tid < 4) {
             const int h = tid - 2, g = h ^ 1;
-            const TauSums q = tau_solve_line(N, h, lu, tab + kTabU * N, sc[kScU + h], none,
-                                             [&](int k) { return -c * s * p1[k]; }, E + 3 * N, z1, 0.0);
+            const TauSums q = tau_solve_line<ANY>(N, h, lu, tab + kTabU * N, sc[kScU + h], none,
+                                                  [&](int k) { return -c * s * p1[k]; }, E, z1, 0.0);
             const double tz = g == PL ? q.psi * s / (2.0 * (N - 1)) + p1[N - 1] * c * s * s * lu.ibeta : 0.0;
             q1 = s * q.k2 + tz;
             sc[kScTz + g] = tz;
@@ -263,9 +345,13 @@ static __global__ __launch_bounds__(64) void k_tau_setup(TauSys t) {
             }
             sc[kScTz + g] = g == PL ? kh * x1[N - 1] : 0.0;
         }
-        if (tid >= 2 && tid < 4) sc[kScQ + ((tid - 2) ^ 1)] = 1.0 / q1;
+        if (tid >= 2 && tid < 4) {
+            sc[kScQ + ((tid - 2) ^ 1)] = 1.0 / q1;
+            if (ANY && q1 == 0.0) atomicOr(&bad, 4);
+        }
         __syncthreads();
     }
+    if (ANY && tid == 0) t.info[key] = bad;
     const int S = tau_row(t.shape);
     double* out = t.table + (size_t)key * tau_table_stride(t.shape);
     for (int i = tid; i < 6 * S; i += 64) {
@@ -442,7 +528,7 @@ struct TauArgs {
     const double2* bcv;   // [2 mode + w]: b on wall w (0: z = 0, 1: z = Lz) at the mode
     const int2* modes;    // 3-D: (mode, key), sorted by key
     const double* rot;    // 3-D: (cos, sin) of the k_h direction per mode
-    int psi;              // some key uses the psi-form
+    int form;             // TauForm
     const cplx<T>*R1, *R2, *R3x, *R3y, *R3z;  // right-hand-side rows, mode-major (R1 null: zero)
     cplx<T>*P, *B, *UX, *UY, *UZ, *taus;
 };
@@ -460,6 +546,14 @@ template <int G, int E>
 constexpr size_t tau_park_bytes() {  // 3-D: the perp row of both waves
     return (size_t)128 * E * sizeof(double2);
 }
+template <int E, int FORM>
+constexpr size_t tau_any_bytes() {  // any sign: tau_bordered's rows of both waves, two parts each
+    return FORM == kTauAny ? (size_t)4 * 64 * E * 5 * sizeof(double) : 0;
+}
+template <int G, int E, bool THREE, int FORM>
+constexpr size_t tau_lds_bytes() {  // of one pair of waves
+    return tau_pair_bytes<G, E>() + (THREE ? tau_park_bytes<G, E>() : 0) + tau_any_bytes<E, FORM>();
+}
 
 // One pair of waves: 64 / G modes, `slot0` the first; wave g holds the degrees of parity g, all rows in
 // registers ([degree][part]).  LDS turns the rows between the memory order (neighbouring lanes,
@@ -470,11 +564,11 @@ constexpr size_t tau_park_bytes() {  // 3-D: the perp row of both waves
 // 2-D: the latency of one wave's instructions, whose fetch is part of it, as the code runs once; a wave
 // per parity halves it against one wave for both (1024 x 256 FP32: 13.7 against 24.4 us, and 200 us with
 // dense inverses; 320 x 97 FP64: 7.6, 19.7 and 19.4 us).
-template <typename T, bool THREE, int G, int E, bool PSI, bool HASD, bool MEAN>
+template <typename T, bool THREE, int G, int E, int FORM, bool HASD, bool MEAN>
 __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const TauArgs<T>& s, int slot0, int g, unsigned char* lds) {
 #pragma clang fp contract(off)
     using V = cplx<T>;
-    constexpr bool LOW = sizeof(T) == 8;  // tau_low_kh
+    constexpr bool ANY = FORM == kTauAny, PSI = FORM != kTauU, LOW = sizeof(T) == 8;
     constexpr int NM = 64 / G, K = 2 * E, LS = (K + 1) * G;  // LDS: K + 1 values per lane, so lanes differ in bank
     const int lane = (int)threadIdx.x & 63, l = lane & (G - 1), grp = lane / G;
     const int N = s.t.N, S = K * G, k0 = K * l + g;  // own degrees: k0 + 2 i
@@ -575,7 +669,7 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
     auto coeff = [&](int r, int i) { return AHEAD ? cof[AHEAD ? r : 0][i] : co[r * S + 2 * i * G]; };
     auto line_of = [&](int op) {
         const double* q = sc + kScLine + 4 * op;
-        return TauLine{q[0], q[1], q[2], q[3], q[0] > s.t.bound};
+        return TauLine{q[0], q[1], q[2], q[3], fabs(q[0]) > s.t.bound};
     };
     // ---- right-hand sides ----
     Row b, x, z;
@@ -618,12 +712,15 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
             d[i][1] *= ic;
         }
     }
+    double* const bordered = reinterpret_cast<double*>(lds + tau_pair_bytes<G, E>() + (THREE ? tau_park_bytes<G, E>() : 0)) +
+                             2 * 64 * E * 5 * g;  // any sign only
     // One line (real and imaginary part) of an operator: r at the own degrees, G = gs Go of the other parity;
     // the result over r.  w = wall sums; tops receives r at N - 1 (A) or psi at N - 2 (B).
     auto line = [&](auto hasg, const TauLine& L, const double (&a)[E], double iW, Row& r, const Nbr& Go, double gs,
                     const double (&w)[2], double (&tops)[2]) __attribute__((always_inline)) {
         if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);  // one line at a time: interleaved, their registers would spill
         constexpr bool HASG = decltype(hasg)::value;
+        const bool piv = ANY && !(L.m > 0.0);  // the same in the whole workgroup, which has one mode
         double e[2][E], e1[PSI ? 2 : 1][PSI ? E : 1], h[E], pr[E];
         {
             double t1[E], t2[E], g1[HASG || PSI ? E : 1], g2[HASG ? E : 1];
@@ -652,36 +749,64 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
                         v = L.psi ? vp : v;
                     }
                     e[p][i] = -(a[i] * L.ial) * v;
+                    if constexpr (ANY) {
+                        const int k = k0 + 2 * i;
+                        if (piv) e[p][i] = k >= 2 && k < N ? -(tau_lo(k) * L.ibeta) * v : 0.0;
+                    }
                 }
             }
         }
-        tau_scan_down<G, E, 2>(h, e, l);
-        if (l == 0) e[0][0] = e[1][0] = 0.0;
+        if (!piv) {
+            tau_scan_down<G, E, 2>(h, e, l);
+            if (l == 0) e[0][0] = e[1][0] = 0.0;
+        }
         if constexpr (PSI)
 #pragma unroll
             for (int p = 0; p < 2; ++p)
 #pragma unroll
                 for (int i = 0; i < E; ++i) e1[p][i] = e[p][i];
-        tau_scan_up<G, E, 2>(a, e, pr, l);
+        if (!piv) tau_scan_up<G, E, 2>(a, e, pr, l);
+        double wts[2];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-            double sum = 0.0, rs = 0.0;
-#pragma unroll
-            for (int i = 0; i < E; ++i) {
-                sum += e[p][i];
-                if (PSI && k0 + 2 * i != N - 1) rs += r[i][p];
-            }
-            sum = lanes_sum<G>(sum);
-            double wt = w[p];
+            double rs = 0.0;
+            wts[p] = w[p];
             if (PSI) {
+#pragma unroll
+                for (int i = 0; i < E; ++i)
+                    if (k0 + 2 * i != N - 1) rs += r[i][p];
                 rs = lanes_sum<G>(rs);
-                if (L.psi) wt = L.m * wt - rs * L.ibeta;
+                if (L.psi) wts[p] = L.m * wts[p] - rs * L.ibeta;
             }
-            const double x0 = (wt - sum) * iW;
+        }
+        if (ANY && piv) {  // lane p solves part p, row by row
+            double* S[2] = {bordered, bordered + 64 * E * 5};
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int i = 0; i < E; ++i) S[p][5 * (E * l + i) + 4] = e[p][i];
+            __syncthreads();
+            if (l < 2) tau_bordered(N, g, L.m, l == 0 ? wts[0] : wts[1], l == 0 ? S[0] : S[1]);
+            __syncthreads();
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int i = 0; i < E; ++i) e[p][i] = k0 + 2 * i < N ? S[p][5 * (E * l + i) + 4] : 0.0;
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            double x0 = 0.0;
+            if (!piv) {
+                double sum = 0.0;
+#pragma unroll
+                for (int i = 0; i < E; ++i) sum += e[p][i];
+                x0 = (wts[p] - lanes_sum<G>(sum)) * iW;
+            }
+            const double below = ANY ? lane_below<G>(e[p][E - 1], l) : 0.0;  // degree k0 - 2
             double uu[E], rt = 0.0, vt = 0.0;
 #pragma unroll
             for (int i = 0; i < E; ++i) {
-                const double v = fma(pr[i], x0, e[p][i]);
+                const double v = piv ? e[p][i] : fma(pr[i], x0, e[p][i]);
                 rt = k0 + 2 * i == kt ? r[i][p] : rt;
                 vt = k0 + 2 * i == kt ? v : vt;
                 e[p][i] = v;
@@ -699,17 +824,19 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
                 for (int i = 0; i < E; ++i) {
                     const int k = k0 + 2 * i;
                     const bool in = k < N - 1;
-                    ab[0][i] = in ? fabs(e[p][i]) : 0.0;
+                    if (piv) ab[0][i] = k == N - 1 ? fabs(L.m * (i > 0 ? e[p][i > 0 ? i - 1 : 0] : below)) * tau_lo(k) : 0.0;
+                    else ab[0][i] = in ? fabs(e[p][i]) : 0.0;
                     su += in ? uu[i] : 0.0;
                     sa += in ? fabs(uu[i]) : 0.0;
                     if (k == N - 1) lo = fabs(e1[p][PSI ? i : 0]);
                 }
-                tau_scan_up<G, E, 1>(a, ab, q, l);
+                if (!piv) tau_scan_up<G, E, 1>(a, ab, q, l);
                 su = lanes_sum<G>(su);
                 sa = lanes_sum<G>(sa);
 #pragma unroll
                 for (int i = 0; i < E; ++i)
-                    if (k0 + 2 * i == N - 1 && L.psi && (ab[0][i] + lo) * L.beta * L.ial > sa + fabs(w[p])) uu[i] = w[p] - su;
+                    if (k0 + 2 * i == N - 1 && L.psi && (ab[0][i] + lo) * fabs(L.beta * L.ial) > sa + fabs(w[p]))
+                        uu[i] = w[p] - su;
             }
 #pragma unroll
             for (int i = 0; i < E; ++i) r[i][p] = uu[i];  // beyond N - 1 a, e and r are zero
@@ -1016,30 +1143,30 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
 }
 
 // the workgroup with the kh = 0 mode (key 0 sorts first) has a body of its own
-template <typename T, bool THREE, int G, int E, bool PSI, bool HASD>
+template <typename T, bool THREE, int G, int E, int FORM, bool HASD>
 __device__ __attribute__((always_inline)) inline void tau_solve_pair(const TauArgs<T>& s, int slot0, bool first, int g,
                                                                       unsigned char* lds) {
-    if (first) tau_solve_pair_t<T, THREE, G, E, PSI, HASD, true>(s, slot0, g, lds);
-    else tau_solve_pair_t<T, THREE, G, E, PSI, HASD, false>(s, slot0, g, lds);
+    if (first) tau_solve_pair_t<T, THREE, G, E, FORM, HASD, true>(s, slot0, g, lds);
+    else tau_solve_pair_t<T, THREE, G, E, FORM, HASD, false>(s, slot0, g, lds);
 }
 
 // 3-D: the pairs of a workgroup have modes of their own; one or two of them give the same bits.
-// Dynamic LDS: tau_pair_bytes + tau_park_bytes per pair.
-template <typename T, int G, int E, bool PSI, bool HASD>
+// Dynamic LDS: tau_lds_bytes per pair.
+template <typename T, int G, int E, int FORM, bool HASD>
 __global__ __launch_bounds__(256, 2) void k3_tau_solve(TauArgs<T> s) {
     extern __shared__ unsigned char smem_raw[];
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), pair = w >> 1;
     const int slot = ((int)blockIdx.x * ((int)blockDim.x >> 7) + pair) * (64 / G);
-    tau_solve_pair<T, true, G, E, PSI, HASD>(s, slot, blockIdx.x == 0, w & 1, 
-                                             smem_raw + pair * (tau_pair_bytes<G, E>() + tau_park_bytes<G, E>()));
+    tau_solve_pair<T, true, G, E, FORM, HASD>(s, slot, blockIdx.x == 0, w & 1,
+                                              smem_raw + pair * tau_lds_bytes<G, E, true, FORM>());
 }
 
 // 2-D: one pair per workgroup
-template <typename T, int G, int E, bool PSI, bool HASD>
+template <typename T, int G, int E, int FORM, bool HASD>
 __global__ __launch_bounds__(128) void k_ch_tau_solve(TauArgs<T> s) {
-    __shared__ double2 lds[tau_pair_bytes<G, E>() / sizeof(double2)];
+    __shared__ double2 lds[tau_lds_bytes<G, E, false, FORM>() / sizeof(double2)];
     const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    tau_solve_pair<T, false, G, E, PSI, HASD>(s, (int)blockIdx.x * (64 / G), blockIdx.x == 0, g,
+    tau_solve_pair<T, false, G, E, FORM, HASD>(s, (int)blockIdx.x * (64 / G), blockIdx.x == 0, g,
                                               reinterpret_cast<unsigned char*>(lds));
 }
 
@@ -1051,7 +1178,7 @@ struct TauItem {
     TauArgs<T> s;
     int wg0;
 };
-template <typename T, bool PSI, bool HASD>
+template <typename T, int FORM, bool HASD>
 __global__ __launch_bounds__(128) void k_ch_tau_solve_group(const TauItem<T>* __restrict__ items, int nitems) {
     __shared__ double2 lds[tau_pair_bytes<64, 4>() / sizeof(double2)];  // the largest shape's
     const int w = (int)blockIdx.x;
@@ -1065,29 +1192,36 @@ __global__ __launch_bounds__(128) void k_ch_tau_solve_group(const TauItem<T>* __
     const int wg = w - items[lo].wg0, g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     unsigned char* const mem = reinterpret_cast<unsigned char*>(lds);
     switch (tau_row(s.t.shape)) {  // the 2-D shapes of tau_shape
-        case 64: tau_solve_pair<T, false, 32, 1, PSI, HASD>(s, 2 * wg, wg == 0, g, mem); break;
-        case 128: tau_solve_pair<T, false, 64, 1, PSI, HASD>(s, wg, wg == 0, g, mem); break;
-        case 256: tau_solve_pair<T, false, 64, 2, PSI, HASD>(s, wg, wg == 0, g, mem); break;
-        default: tau_solve_pair<T, false, 64, 4, PSI, HASD>(s, wg, wg == 0, g, mem); break;
+        case 64: tau_solve_pair<T, false, 32, 1, FORM, HASD>(s, 2 * wg, wg == 0, g, mem); break;
+        case 128: tau_solve_pair<T, false, 64, 1, FORM, HASD>(s, wg, wg == 0, g, mem); break;
+        case 256: tau_solve_pair<T, false, 64, 2, FORM, HASD>(s, wg, wg == 0, g, mem); break;
+        default: tau_solve_pair<T, false, 64, 4, FORM, HASD>(s, wg, wg == 0, g, mem); break;
     }
 }
 
-// f(psi, has R1) with the two flags as compile-time constants
+// f(form, has R1) with both as compile-time constants; f's any-sign kernels are launched by the caller
 template <typename F>
-inline void tau_flags(bool psi, bool hasd, F&& f) {
+inline void tau_flags(int form, bool hasd, F&& f) {
     using yes = std::true_type;
     using no = std::false_type;
-    if (psi && hasd) f(yes{}, yes{});
-    else if (psi) f(yes{}, no{});
-    else if (hasd) f(no{}, yes{});
-    else f(no{}, no{});
+    using psi = std::integral_constant<int, kTauPsi>;
+    using u = std::integral_constant<int, kTauU>;
+    if (form == kTauPsi && hasd) f(psi{}, yes{});
+    else if (form == kTauPsi) f(psi{}, no{});
+    else if (hasd) f(u{}, yes{});
+    else f(u{}, no{});
 }
 
-// whether any key up to kh_max takes the psi-form
-inline bool tau_uses_psi(const TauSys& t, double kh_max) {
+// the recursion of the keys up to kh_max: kTauPsi when any line among them takes the psi-form
+inline int tau_form(const TauSys& t, double kh_max) {
+    if (tau_any_sign(t.kappa, t.nu)) return kTauAny;
     const double k2 = kh_max * kh_max / (t.s * t.s);  // m of the pressure lines, below those of b and u
     const double mb = 1.0 / (t.c * t.kappa * t.s * t.s) + k2, mu = 1.0 / (t.c * t.nu * t.s * t.s) + k2;
-    return mb > t.bound || mu > t.bound;
+    return mb > t.bound || mu > t.bound ? kTauPsi : kTauU;
 }
+
+// whether the equation of a diffusivity has lost it (the D T_{N-1} lift is left without a coefficient): zero, or
+// too small for FP64
+inline bool tau_no_diffusion(double c, double s, double diff) { return std::isinf(1.0 / (c * diff * s * s)); }
 
 }  // namespace tarang

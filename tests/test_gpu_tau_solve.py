@@ -13,10 +13,13 @@ is what an equation row leaves over, whose terms reach (1/dt + nu (2/Lz)^2 N^4) 
 import numpy as np
 import pytest
 
+from tarang_amd import _lib
 from tarang_amd._lib import CHAN3_B, CHAN3_P, CHAN3_UX, CHAN3_UY, CHAN3_UZ, CHAN_B, CHAN_P, CHAN_UX, CHAN_UZ
+from tests.conftest import relerr
 from tests.tau_reference import Mode
 from tests.test_gpu_channel import random_state
 from tests.test_gpu_channel3d import random_state3
+from tests.test_gpu_channel_group import make_group
 
 pytestmark = pytest.mark.gpu
 
@@ -161,3 +164,123 @@ def test_tau_solve_precision_3d(gpu, N, mr):
                 err[f].append(float(np.linalg.norm((got[f] - ref[f]).astype(float)) / size))
                 lu[f].append(float(np.linalg.norm((dense[f] - ref[f]).astype(float)) / size))
     check_precision(err, lu, "3-D")
+
+
+def zero_pivot(N, g):
+    """A negative m at which elimination from the top degree down without pivoting meets a zero pivot."""
+    def smallest(m):  # the pivots' running product changes sign where one of them does
+        top = (N - 1) % 2 == g
+        an, out = 0.0, []
+        for j in range((N + 1 - g) // 2 - (2 if top else 1), 0, -1):
+            k = 2 * j + g
+            lo = (2.0 if k == 2 else 1.0) / (4.0 * k * (k - 1))
+            if k == N - 2:
+                den = 1.0 + m * lo * (0.5 if k == 2 else 1.0)
+            else:
+                den = 1.0 + m / (2.0 * (k * k - 1.0)) - (0.0 if k == N - 3 else m / (4.0 * k * (k + 1)) * an)
+            an = m * lo / den
+            out.append(den)
+        return min(out)
+
+    a = -1.0
+    while smallest(2 * a) > 0:
+        a *= 2
+    b = 2 * a
+    for _ in range(200):
+        c = 0.5 * (a + b)
+        a, b = (c, b) if smallest(c) > 0 else (a, c)
+    return a
+
+
+ANY_SIGN = [("zero", "zero"), (-1e-2, -3e-3), (-1e-2, 1e-3), (1e-3, -1e-3)]  # kappa, nu
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kappa,nu", ANY_SIGN)
+@pytest.mark.parametrize("N", [9, 33, 64, 128])
+def test_tau_solve_any_sign_2d(gpu, N, kappa, nu, dtype):
+    """Negative diffusivities, "zero" among them: a value that brings a pivot of the unpivoted recursion to
+    zero in the mean mode.  Against long double: 1e-10 (a line is good to 1e-13, and uz is what up to a
+    hundredth of the pressure gradient's size leaves), 1e-6 for the rounding of an FP32 result."""
+    print(f"tau solve any sign 2-D N={N} kappa={kappa} nu={nu} {dtype.__name__}", flush=True)
+    nx, Lx, Lz, dt = 8, 4.0, 1.0, 2.0 ** -10
+    if kappa == "zero":
+        kappa = nu = 1.0 / (zero_pivot(N, N % 2) * dt * 4.0)
+    scale, tol = (SCALE, 1e-10) if dtype == np.float64 else (2.0 ** -75, 1e-6)
+    rng = np.random.default_rng(N)
+    st = {v: spectrum(rng, (nx // 2 + 1, N), N).astype(np.complex64 if dtype == np.float32 else complex)
+          for v in (CHAN_B, CHAN_UX, CHAN_UZ)}
+    for c in st.values():
+        c[[0, -1]] = c[[0, -1]].real
+    s = gpu.chan(nx, N, Lx, Lz, kappa, nu, dt, stepper=4, dtype=dtype, b_bottom=0.0, b_top=0.0)
+    for v, c in st.items():
+        s.set(v, c * c.real.dtype.type(scale))
+    s.step(1)
+    got = {f: s.get(v).astype(complex) / scale for f, v in (("b", CHAN_B), ("u", CHAN_UX), ("uz", CHAN_UZ), ("p", CHAN_P))}
+    s.close()
+    for m in range(nx // 2):
+        st64 = {v: c[m].astype(complex) for v, c in st.items()}
+        ref = Mode(N, 2 * np.pi * m / Lx, dt, kappa, nu, 2.0 / Lz)(
+            parts(st64[CHAN_B]), parts(-1j * st64[CHAN_UX]), parts(st64[CHAN_UZ]))
+        for f in got:
+            g = parts(-1j * got[f][m] if f == "u" else got[f][m])
+            size = max(float(np.linalg.norm(ref[f].astype(float))), 1e-3 * float(np.linalg.norm(ref["u"].astype(float))))
+            e = float(np.linalg.norm((g - ref[f]).astype(float))) / size
+            assert e <= tol, (m, f, e)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ts", ["SBDF2", "RK222"])
+@pytest.mark.parametrize("N", [6, 33, 256])
+def test_tau_solve_any_sign_steps(gpu, oracle, N, ts, dtype):
+    """Steps with negative diffusivities against the oracle's dense LU, in 2-D, 3-D and as a group member.  The
+    oracle multiplies a relative change of the state by up to 40 here (400 in one FP64 case): 40 times the 1e-5
+    of other FP32 steps, and 1e-9 for their 1e-12."""
+    print(f"tau solve any sign steps N={N} {ts} {dtype.__name__}", flush=True)
+    tol = 1e-9 if dtype == np.float64 else 4e-4
+    kappa, nu, dt, code = -1e-3, -2e-3, 1e-3, {"RK222": 0, "SBDF2": 2}[ts]
+    st = random_state(oracle, 16, N, 4.0, 1.0, seed=N)
+    pair = [oracle.RBC2D(16, N, 4.0, 1.0, kappa, nu, dt, ts)]
+    pair += [gpu.chan(16, N, 4.0, 1.0, kappa, nu, dt, stepper=code, dtype=dtype) for _ in range(2)]
+    other = [gpu.chan(16, 33, 4.0, 1.0, 1e-3, 1e-3, dt, stepper=code, dtype=dtype) for _ in range(2)]
+    for s in pair:
+        for v, c in st.items():
+            s.set(v, c)
+    for s in other:
+        for v, c in random_state(oracle, 16, 33, 4.0, 1.0, seed=1).items():
+            s.set(v, c)
+    ref, s, member = pair
+    ref.step(2)
+    s.step(2)
+    g = make_group([member, other[0]])
+    _lib.call("tarang_chan_group_step", g, 2)
+    gpu.sync()
+    other[1].step(2)
+    for v in (oracle.RBC_B, oracle.RBC_UX, oracle.RBC_UZ):
+        assert relerr(s.get(v), ref.get(v)) < tol, v
+        assert np.array_equal(member.get(v), s.get(v)) and np.array_equal(other[0].get(v), other[1].get(v))
+    _lib.call("tarang_chan_group_destroy", g)
+    for x in pair[1:] + other:
+        x.close()
+    if N > 64:
+        return
+    st, _ = random_state3(oracle, 8, 8, N, 4.0, 3.0, 1.0, seed=N)
+    ref = oracle.RBC3D(8, 8, N, 4.0, 3.0, 1.0, kappa, nu, dt, ts)
+    s = gpu.chan3(8, 8, N, 4.0, 3.0, 1.0, kappa, nu, dt, stepper=code, dtype=dtype)
+    for v, c in st.items():
+        ref.set(v, c)
+        s.set(v, c)
+    ref.step(2)
+    s.step(2)
+    for v in (oracle.RBC3_B, oracle.RBC3_UX, oracle.RBC3_UY, oracle.RBC3_UZ):
+        assert relerr(s.get(v), ref.get(v)) < tol, v
+    s.close()
+
+
+def test_tau_solve_without_diffusion_is_singular(gpu):
+    """Zero, and a diffusivity that FP64 cannot divide by."""
+    for kappa, nu in ((0.0, 1e-3), (1e-3, 0.0), (1e-320, 1e-3), (1e-3, -1e-320)):
+        for make in (lambda: gpu.chan(16, 9, 4.0, 1.0, kappa, nu, 1e-3), lambda: gpu.chan3(8, 8, 9, 4.0, 4.0, 1.0, kappa, nu, 1e-3)):
+            with pytest.raises(_lib.TarangError) as e:
+                make()
+            assert e.value.code == _lib.ERR_SINGULAR and "singular" in str(e.value)
