@@ -71,7 +71,7 @@ class Device:
 
     def chan(self, nx, nz, Lx, Lz, kappa, nu, dt, stepper=0, dtype=np.float64, b_bottom=None, b_top=0.0, refine=0,
              split=None):
-        """split=None: the library's recommended form (split inverses for an FP32 state)."""
+        """split=None: split_inverse as the Python API sets it (1 for an FP32 state); it has no effect."""
         d = _lib.ChanDesc()
         d.refine_sweeps = refine
         d.split_inverse = (1 if dtype == np.float32 else 0) if split is None else split

@@ -12,7 +12,7 @@ LD = np.longdouble
 
 
 def solve(A, B, dtype=LD):
-    """Gaussian elimination with partial pivoting in `dtype`, column scaling-free; B is (n, m)."""
+    """Gaussian elimination with partial pivoting in `dtype`; B is (n, m)."""
     A, B = A.astype(dtype).copy(), B.astype(dtype).copy()
     n = len(A)
     for k in range(n):
@@ -27,6 +27,16 @@ def solve(A, B, dtype=LD):
     for k in range(n - 1, -1, -1):
         B[k] = (B[k] - A[k, k + 1:] @ B[k + 1:]) / A[k, k]
     return B
+
+
+def solve_by_parity(A, B, rows, cols, dtype):
+    """The two decoupled halves of A X = B: rows and cols label every equation and unknown 0 or 1."""
+    X = np.zeros((len(cols), B.shape[1]), dtype)
+    for q in (0, 1):
+        r, c = np.flatnonzero(rows == q), np.flatnonzero(cols == q)
+        assert not A[np.ix_(r, np.flatnonzero(cols != q))].any()
+        X[c] = solve(A[np.ix_(r, c)], B[r], dtype)
+    return X
 
 
 def deriv(N, s):
@@ -47,7 +57,11 @@ class Mode:
         D = deriv(N, s)
         D2, I = D @ D, np.eye(N, dtype=LD)
         self.last, self.dlast = I[:, N - 1], D[:, N - 1]
-        self.walls = np.stack([(LD(-1)) ** np.arange(N), np.ones(N, LD)])
+        k = np.arange(N)
+        self.walls = np.stack([k % 2 == 0, k % 2 == 1]).astype(LD)  # half the sum and difference of the wall values
+        top = np.array([(N - 2) % 2, (N - 1) % 2])  # degrees of D T_{N-1} and T_{N-1}
+        self.rb = np.concatenate([k % 2, [0, 1]])
+        self.cb = np.concatenate([k % 2, top])
 
         def helm(diff):
             return (1 + c * LD(diff) * kh * kh) * I - c * LD(diff) * D2
@@ -60,7 +74,7 @@ class Mode:
             return A
 
         self.Ab, self.Ay = scalar(kappa), scalar(nu)
-        mean = kh == 0
+        mean = bool(kh == 0)
         n = 3 * N + 4 + (1 if mean else 0)
         A = np.zeros((n, n), LD)
         X, P, Z, t = slice(0, N), slice(N, 2 * N), slice(2 * N, 3 * N), 3 * N
@@ -72,9 +86,11 @@ class Mode:
         A[P, t + 2] = c * self.last
         A[t:t + 2, X] = self.walls
         A[t + 2:t + 4, Z] = self.walls
+        # halves by the parity of u~ and p; uz and E3z have the other one
+        self.ru = np.concatenate([k % 2, k % 2, 1 - k % 2, [0, 1, 1, 0], [0] * mean])
+        self.cu = np.concatenate([k % 2, k % 2, 1 - k % 2, top, 1 - top, [0] * mean])
         if mean:  # tau_p in the constant row of E1, integ(p) = 0
             A[N, t + 4] = c
-            k = np.arange(N)
             A[t + 4, P] = np.where(k % 2 == 0, LD(1) / (1 - k.astype(LD) ** 2 + (k == 1)), 0)
         self.A = A
 
@@ -83,14 +99,14 @@ class Mode:
         N, d = self.N, self.dtype
         m = rb.shape[1]
         z2 = np.zeros((2, m), LD)
-        ob = solve(self.Ab, np.concatenate([rb, z2]), d)
+        ob = solve_by_parity(self.Ab, np.concatenate([rb, z2]), self.rb, self.cb, d)
         rhs = np.zeros((len(self.A), m), LD)
         rhs[:N] = rx
         rhs[2 * N:3 * N] = rz + self.c * ob[:N]
-        o = solve(self.A, rhs, d)
+        o = solve_by_parity(self.A, rhs, self.ru, self.cu, d)
         out = {"b": ob[:N], "tau_b1": ob[N], "tau_b2": ob[N + 1], "u": o[:N], "p": o[N:2 * N], "uz": o[2 * N:3 * N],
                "tau_u1": o[3 * N], "tau_u2": o[3 * N + 1], "tau_u1z": o[3 * N + 2], "tau_u2z": o[3 * N + 3]}
         if ry is not None:
-            ov = solve(self.Ay, np.concatenate([ry, z2]), d)
+            ov = solve_by_parity(self.Ay, np.concatenate([ry, z2]), self.rb, self.cb, d)
             out.update({"v": ov[:N], "tau_v1": ov[N], "tau_v2": ov[N + 1]})
         return out

@@ -234,8 +234,8 @@ def test_rbc3d_through_api(oracle):
     # is within 1e-11)
     assert staterr(pairs) < 1e-12 and max(errs[1:]) < 1e-11
     # lift taus are the ill-conditioned components of the per-mode tau systems (condition
-    # numbers up to ~3e7): the GPU applies explicit inverses, the oracle LU solves, and the
-    # two roundings differ there by ~cond x eps relative to the taus' own scale
+    # numbers up to ~3e7): the GPU's line solves and the oracle's LU solves round
+    # differently there, by ~cond x eps relative to the taus' own scale
     assert relerr(tau_b1._c.cpu().numpy().T, ref.tau(1)) < 1e-8
     solver.close()
 
