@@ -237,7 +237,7 @@ struct Ch3SbdfArgs {
     const cplx<T>* F[4];   // F_n rows E2, E3x, E3y, E3z
     cplx<T>* Fm1[4];
     cplx<T>* MXm1[4];
-    cplx<T>* R[5];         // E1, E2, E3x, E3y, E3z
+    cplx<T>* R[4];         // E2, E3x, E3y, E3z (E1: zero)
     T c1, c2, a1, a2, inv_a0;
     Ch3Geom geo;
 };
@@ -250,7 +250,6 @@ __global__ void k3_sbdf(Ch3SbdfArgs<T> a, size_t n) {
         const int m = mode % nxh, nn = mode / nxh;
         const bool xline = m == 0 || ((a.geo.nx % 2) == 0 && m == a.geo.nx / 2);
         const size_t partner = ((size_t)(m + nxh * ((ny - nn) % ny))) * N + k;
-        a.R[0][i] = cplx<T>{T(0), T(0)};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             cplx<T> x = a.X[r][i];
@@ -261,7 +260,7 @@ __global__ void k3_sbdf(Ch3SbdfArgs<T> a, size_t n) {
             const cplx<T> f = a.F[r][i], fo = a.Fm1[r][i], mo = a.MXm1[r][i];
             const T vx = a.c1 * f.x + a.c2 * fo.x - a.a1 * x.x - a.a2 * mo.x;
             const T vy = a.c1 * f.y + a.c2 * fo.y - a.a1 * x.y - a.a2 * mo.y;
-            a.R[r + 1][i] = cplx<T>{vx * a.inv_a0, vy * a.inv_a0};
+            a.R[r][i] = cplx<T>{vx * a.inv_a0, vy * a.inv_a0};
             a.Fm1[r][i] = f;
             a.MXm1[r][i] = x;
         }

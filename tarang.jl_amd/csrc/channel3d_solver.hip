@@ -78,13 +78,13 @@ Channel3Solver::Channel3Solver(Context* ctx, const Channel3Desc& d) : ctx_(ctx),
         zeroed(Fm1_[r], fb);
         zeroed(MXm1_[r], fb);
     }
-    for (int r = 0; r < 5; ++r) zeroed(R_[r], fb);
+    for (int r = multistep() ? 1 : 0; r < 5; ++r) zeroed(R_[r], fb);  // the multistep E1 rows are zero
     tab_ = make_tableau(d.stepper);
     if (!multistep()) {
         for (int r = 0; r < 4; ++r) zeroed(X0_[r], fb);
         for (int st = 0; st < tab_.stages; ++st) {
             for (int r = 0; r < 4; ++r) zeroed(Frk_[st][r], fb);
-            for (int r = 0; r < 5; ++r) zeroed(LX_[st][r], fb);
+            for (int r = 0; r < 5 && uses_lx(tab_, st); ++r) zeroed(LX_[st][r], fb);
         }
     }
     const size_t prow = (size_t)d.nz * my_ * nxh_ * vb;  // one y-padded plane
@@ -460,7 +460,7 @@ void Channel3Solver::sbdf_t(bool first) {
         a.Fm1[r] = Fm1_[r].as<V>();
         a.MXm1[r] = MXm1_[r].as<V>();
     }
-    for (int r = 0; r < 5; ++r) a.R[r] = R_[r].as<V>();
+    for (int r = 0; r < 4; ++r) a.R[r] = R_[r + 1].as<V>();
     a.c1 = T(c1); a.c2 = T(c2); a.a1 = T(a1); a.a2 = T(a2); a.inv_a0 = T(1.0 / a0);
     a.geo = Ch3Geom{d_.nx, d_.ny, nxh_, d_.nz, nmodes_, 2.0 * M_PI / d_.Lx, 2.0 * M_PI / d_.Ly};
     const size_t n = field_elems();
@@ -717,7 +717,7 @@ void Channel3Solver::kernel_bytes(double* out) const {
     out[2] = (kCh3Planes * pad + 4 * pad) * vb;                 // read 12 padded planes, write 4
     out[3] = (4 * pad + 4 * nc) * vb;                           // read 4 padded planes, write 4
     out[4] = (8 * nc) * vb + N * N * rb;                        // read 4 planes, write 4 rows
-    out[5] = (4 * 4 + 4 + 5) * nc * vb;                         // state (x2 on the kx lines), F, histories, rhs
+    out[5] = (4 * 4 + 3 * 4) * nc * vb;                         // read state, F, histories; write histories, rhs
     // solve: rhs rows and the per-key tables in, five fields out
     out[6] = (multistep() ? 9 : 10) * nc * vb +
              (double)nkeys_ * tau_table_stride(tau_shape(d_.nz, true, any_sign())) * sizeof(double);
@@ -735,8 +735,11 @@ size_t footprint(const Channel3Desc& d) {
     const size_t nxh = d.nx / 2 + 1, nmodes = nxh * d.ny, N = d.nz, vb = 2 * dtype_size((DType)d.dtype);
     const size_t fb = nmodes * N * vb, prow = N * (size_t)padded_len(d.ny) * nxh * vb, ib = dtype_size((DType)d.dtype);
     const bool ms = d.stepper == kSBDF2 || d.stepper == kSBDF1;
-    const size_t S = ms ? 0 : (size_t)make_tableau(d.stepper).stages;
-    const size_t nfields = 5 + 12 + 5 + (ms ? 0 : 4 + 9 * S);  // state, history, rhs rows, RK stage rows
+    size_t nfields = 5 + 12 + (ms ? 4 : 5 + 4);  // state, history, rhs rows, RK initial state
+    if (!ms) {
+        const Tableau tab = make_tableau(d.stepper);
+        for (int st = 0; st < tab.stages; ++st) nfields += 4 + (uses_lx(tab, st) ? 5 : 0);  // RK stage rows
+    }
     // distinct |k_h|^2 keys: at most one per mode (about nmodes / 5.6 at 256 x 256 when Lx == Ly)
     const size_t keys = d.Lx == d.Ly ? nmodes / 3 + 64 : nmodes;
     size_t b = nfields * alloc_granule(fb) + alloc_granule(kCh3ZPlanes * fb) + alloc_granule(kCh3Planes * prow) +

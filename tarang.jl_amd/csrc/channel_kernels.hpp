@@ -546,7 +546,7 @@ __global__ void k_ch_stage(ChStageArgs<T> a, size_t n) {
 
 // Per-mode multistep right-hand side (step_subproblem_multistep.jl:197-420), scaled by
 // 1/a0 so that the solve uses M + (1/a0) L:
-//   R = (c1 F_n + c2 F_{n-1} - a1 M P(x_n) - a2 M P(x_{n-1})) / a0,   E1 rows 0
+//   R = (c1 F_n + c2 F_{n-1} - a1 M P(x_n) - a2 M P(x_{n-1})) / a0;   E1 rows 0, not stored
 // M P(x) is the evolved part (b, ux, uz) of the grid-round-tripped state.  The
 // histories F_{n-1}, M P(x_{n-1}) are replaced by the current values in the same pass.
 template <typename T>
@@ -555,7 +555,7 @@ struct ChSbdfArgs {
     const cplx<T>* F[3];   // F_n rows E2, E3x, E3z
     cplx<T>* Fm1[3];
     cplx<T>* MXm1[3];
-    cplx<T>* R[4];         // rhs rows E1, E2, E3x, E3z
+    cplx<T>* R[3];         // rhs rows E2, E3x, E3z (E1: zero)
     T c1, c2, a1, a2, inv_a0;
     int N, nx;
 };
@@ -565,7 +565,6 @@ __global__ void k_ch_sbdf(ChSbdfArgs<T> a, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         const int m = (int)(i / a.N);
         const bool proj = m == 0 || ((a.nx % 2) == 0 && m == a.nx / 2);
-        a.R[0][i] = cplx<T>{T(0), T(0)};
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             cplx<T> x = a.X[r][i];
@@ -573,7 +572,7 @@ __global__ void k_ch_sbdf(ChSbdfArgs<T> a, size_t n) {
             const cplx<T> f = a.F[r][i], fo = a.Fm1[r][i], mo = a.MXm1[r][i];
             const T vx = a.c1 * f.x + a.c2 * fo.x - a.a1 * x.x - a.a2 * mo.x;
             const T vy = a.c1 * f.y + a.c2 * fo.y - a.a1 * x.y - a.a2 * mo.y;
-            a.R[r + 1][i] = cplx<T>{vx * a.inv_a0, vy * a.inv_a0};
+            a.R[r][i] = cplx<T>{vx * a.inv_a0, vy * a.inv_a0};
             a.Fm1[r][i] = f;
             a.MXm1[r][i] = x;
         }

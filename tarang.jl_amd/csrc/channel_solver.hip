@@ -77,10 +77,10 @@ ChannelSolver::ChannelSolver(Context* ctx, const ChannelDesc& d) : ctx_(ctx), d_
     } else {
         for (int st = 0; st < tab_.stages; ++st) {
             for (int r = 0; r < 3; ++r) zeroed(F_[st][r], fb);
-            for (int r = 0; r < 4; ++r) zeroed(LX_[st][r], fb);
+            for (int r = 0; r < 4 && uses_lx(tab_, st); ++r) zeroed(LX_[st][r], fb);
         }
     }
-    for (int r = 0; r < 4; ++r) zeroed(R_[r], fb);
+    for (int r = multistep() ? 1 : 0; r < 4; ++r) zeroed(R_[r], fb);  // the multistep E1 rows are zero
     zeroed(G_, 8 * fb);
     zeroed(H_, 3 * fb);
     std::vector<double> BT, BDT, FT;
@@ -422,7 +422,7 @@ void ChannelSolver::sbdf_t(bool first) {
         a.Fm1[r] = Fm1_[r].as<V>();
         a.MXm1[r] = MXm1_[r].as<V>();
     }
-    for (int r = 0; r < 4; ++r) a.R[r] = R_[r].as<V>();
+    for (int r = 0; r < 3; ++r) a.R[r] = R_[r + 1].as<V>();
     a.c1 = T(c1); a.c2 = T(c2); a.a1 = T(a1); a.a2 = T(a2); a.inv_a0 = T(1.0 / a0);
     a.N = d_.nz;
     a.nx = d_.nx;
@@ -612,8 +612,11 @@ size_t footprint(const ChannelDesc& d) {
     // every buffer the constructor allocates, in 2 MiB pages
     const size_t nxh = d.nx / 2 + 1, N = d.nz, vb = 2 * dtype_size((DType)d.dtype), fb = nxh * N * vb;
     const bool ms = d.stepper == kSBDF2 || d.stepper == kSBDF1;
-    const size_t S = ms ? 0 : (size_t)make_tableau(d.stepper).stages;
-    const size_t nfields = 4 + 3 + 4 + (ms ? 9 : 7 * S);  // state, X0, rhs rows, history or stage rows
+    size_t nfields = 4 + 3 + (ms ? 3 + 9 : 4);  // state, X0, rhs rows, history
+    if (!ms) {
+        const Tableau tab = make_tableau(d.stepper);
+        for (int st = 0; st < tab.stages; ++st) nfields += 3 + (uses_lx(tab, st) ? 4 : 0);  // stage rows
+    }
     const size_t ib = dtype_size((DType)d.dtype);
     size_t b = nfields * alloc_granule(fb) + alloc_granule(8 * fb) + alloc_granule(3 * fb);  // G, H
     b += alloc_granule(nxh * 8 * vb) + 3 * alloc_granule(N * N * ib);                       // taus, tables
