@@ -294,8 +294,8 @@ int tarang_chan_kernel_bytes(tarang_chan_t s, double* bytes6);
 /* Several 2-D channel problems stepped together.  The members share one context, dtype,
  * timestepper, refine_sweeps and split_inverse, and may differ in nx, nz, Lx, Lz, kappa,
  * nu, dt and walls.  Every implicit stage solves all members' per-mode tau systems in one
- * launch (workgroups over the modes of every member), and a group step is one hipGraph
- * replay.  Each member keeps its own clock and history, gives the same bits as when stepped
+ * launch (workgroups over the modes of every member; a member with a negative diffusivity
+ * has a launch of its own), and a group step is one hipGraph replay.  Each member keeps its own clock and history, gives the same bits as when stepped
  * alone, and may still be stepped alone; members must outlive the group.  The reference
  * batches the modes of one problem (src/core/subsystems/mode_batch.jl:522-552); it has no
  * batching across problems. */

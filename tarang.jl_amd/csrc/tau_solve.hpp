@@ -40,8 +40,8 @@
 // (row N - 1: tau_u1z = f_{N-1}), its degree 0 the wall sum, and lambda makes the two agree: for an odd
 // uz the integral's wall sum vanishes, for an even one its degree 0 is that of the E3z line.
 //
-// A solve reads the right-hand-side rows and 6 N doubles per |k_h| key and writes the solution
-// (3-D 256 x 256 x 128: 0.33 GB in FP32); the set-up is one small kernel.
+// A solve reads the right-hand-side rows and 6 N doubles per |k_h| key and writes the solution (3-D 256 x 256 x 128:
+// 0.34 GB in FP32, 0.65 GB in FP64; measured 0.38 and 0.70); the set-up is one small kernel.
 #pragma once
 #include <cmath>
 #include <type_traits>
@@ -50,11 +50,16 @@
 
 namespace tarang {
 
+// From which |m| on the psi-form takes u_{N-1} (A) from the wall sum's remainder, which rounds with sum |u|, and
+// not from the recursion, whose amplitudes pass through a_{N-1} = m/(4 N^2).  Over N = 9 .. 256 and m = 0.2 N^2 ..
+// 1e5 N^2 the mean errors are those of a choice by running error sums, which take a scan per line.
+__host__ __device__ inline double tau_rest_bound(int N) { return 64.0 * N * N; }
 // Where the psi-form starts, as a bound on |m|.  FP64: at N^2/8, where the two are equally far from a
 // long-double solve (N = 128: 2e-16 and 1e-16 of the line's 2-norm at m = N^2/20, 4e-16 and 1e-16 at
-// 16 N^2, 1e-15 and 2e-16 at 1000 N^2; a dense LU 2e-16).  FP32 rounds the result at 6e-8, and the psi-form
-// keeps r and a rounding estimate in registers beside the recursion: it starts where the u-form's
-// u_{N-1}, which loses m/(4 N^2) eps |u_{N-3}|, would lose 4 eps (64 from 64 degrees on).
+// 16 N^2, 1e-15 and 2e-16 at 1000 N^2; a dense LU 2e-16); with uz from E1 (below) the psi-form costs 256 x 256 x
+// 128 188 -> 210 us and 320 x 97 7.4 -> 9.4 us, at m = 20 .. 45 N^2.  FP32 rounds the result at 6e-8, and the psi-form
+// keeps r in registers beside the recursion: it starts where the u-form's u_{N-1}, which loses
+// m/(4 N^2) eps |u_{N-3}|, would lose 4 eps (64 from 64 degrees on).
 inline double tau_psi_bound(int N, bool fp64) { return (fp64 ? 0.125 : N < 64 ? 16.0 : 256.0) * N * N; }
 // Up to which kh uz is the integral of E1, in units of s; -1: never.  Against long-double solves at N = 128
 // and m = 30 N^2 / 1000 N^2, uz from E3z / from E1 / by a dense inverse is off by 5e-14 / 1e-15 / 1e-15 and
@@ -230,8 +235,9 @@ __host__ __device__ inline TauSums tau_solve_line(int N, int g, const TauLine& L
         }
         rs += rr(k);
     }
-    const double wt = L.psi ? L.m * w - rs * L.ibeta : w, ft = piv ? fabs(e[5 * (n - 1) + 4]) : 0.0;
-    double x = 0.0, est = 0.0, su = 0.0, sa = 0.0;
+    const double wt = L.psi ? L.m * w - rs * L.ibeta : w;
+    const bool rest = A && L.psi && fabs(L.m) > tau_rest_bound(N);
+    double x = 0.0, su = 0.0;
     TauSums out{0.0, 0.0};
     if (piv) out.ok = tau_bordered(N, g, L.m, wt, e);
     else x = (wt - sum) * iW;
@@ -240,16 +246,8 @@ __host__ __device__ inline TauSums tau_solve_line(int N, int g, const TauLine& L
         if (piv) x = e[5 * j + 4];
         else if (j > 0) x = a[k] * x + e[k];
         double v = L.psi ? (L.beta * x + rr(k)) * L.ial : x;
-        if (L.psi && A) {  // u_{N-1}: the wall sum's remainder where the recursion has lost more
-            if (k < N - 1) {
-                est = (piv || j == 0 ? 0.0 : a[k] * est) + fabs(x);
-                su += v;
-                sa += fabs(v);
-            } else if ((piv ? fabs(L.m) * tau_lo(k) * est + ft : a[k] * est + fabs(e[k])) * fabs(L.beta * L.ial) >
-                       sa + fabs(w)) {
-                v = w - su;
-            }
-        }
+        if (rest && k == N - 1) v = w - su;
+        su += v;
         u[k] = v;
         out.k2 += (double)k * k * v;
     }
@@ -559,11 +557,12 @@ constexpr size_t tau_lds_bytes() {  // of one pair of waves
 // registers ([degree][part]).  LDS turns the rows between the memory order (neighbouring lanes,
 // neighbouring degrees) and a lane's run, and passes G of the other parity.  Every workgroup meets the
 // same barriers: a pair beyond the last mode runs along without storing.
-// Bound: 3-D FP64 issue and HBM alike (256 x 256 x 128 FP32: 0.33 GB in 150 us, 187 us for FP64; dense
-// inverses on the matrix cores read 3.2 / 5.1 GB in 787 / 1262 us; 96 x 80 x 49 FP64 20 against 89 us).
-// 2-D: the latency of one wave's instructions, whose fetch is part of it, as the code runs once; a wave
-// per parity halves it against one wave for both (1024 x 256 FP32: 13.7 against 24.4 us, and 200 us with
-// dense inverses; 320 x 97 FP64: 7.6, 19.7 and 19.4 us).
+// Bound: 3-D, latency: at 256 registers two waves share a SIMD, and each waits for memory or LDS half of its
+// cycles and issues vector instructions a fifth of them (256 x 256 x 128: 151 us at 2.5 TB/s in FP32, 210 us at
+// 3.3 TB/s in FP64, of 5.1 that a copy reaches; dense inverses on the matrix cores read 3.2 / 5.1 GB in 787 /
+// 1262 us; 96 x 80 x 49 FP64 18 against 89 us).  2-D: the latency of one wave's instructions, whose fetch is part
+// of it, as the code runs once; a wave per parity halves it against one wave for both (1024 x 256 FP32: 13.7
+// against 24.4 us, and 200 us with dense inverses; 320 x 97 FP64: 9.4 us, 19.4 with dense inverses).
 template <typename T, bool THREE, int G, int E, int FORM, bool HASD, bool MEAN>
 __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const TauArgs<T>& s, int slot0, int g, unsigned char* lds) {
 #pragma clang fp contract(off)
@@ -721,7 +720,8 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
         if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);  // one line at a time: interleaved, their registers would spill
         constexpr bool HASG = decltype(hasg)::value;
         const bool piv = ANY && !(L.m > 0.0);  // the same in the whole workgroup, which has one mode
-        double e[2][E], e1[PSI ? 2 : 1][PSI ? E : 1], h[E], pr[E];
+        const bool rest = PSI && L.psi && fabs(L.m) > tau_rest_bound(N);
+        double e[2][E], h[E], pr[E];
         {
             double t1[E], t2[E], g1[HASG || PSI ? E : 1], g2[HASG ? E : 1];
 #pragma unroll
@@ -760,11 +760,6 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
             tau_scan_down<G, E, 2>(h, e, l);
             if (l == 0) e[0][0] = e[1][0] = 0.0;
         }
-        if constexpr (PSI)
-#pragma unroll
-            for (int p = 0; p < 2; ++p)
-#pragma unroll
-                for (int i = 0; i < E; ++i) e1[p][i] = e[p][i];
         if (!piv) tau_scan_up<G, E, 2>(a, e, pr, l);
         double wts[2];
 #pragma unroll
@@ -802,7 +797,6 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
                 for (int i = 0; i < E; ++i) sum += e[p][i];
                 x0 = (wts[p] - lanes_sum<G>(sum)) * iW;
             }
-            const double below = ANY ? lane_below<G>(e[p][E - 1], l) : 0.0;  // degree k0 - 2
             double uu[E], rt = 0.0, vt = 0.0;
 #pragma unroll
             for (int i = 0; i < E; ++i) {
@@ -818,25 +812,13 @@ __device__ __attribute__((always_inline)) inline void tau_solve_pair_t(const Tau
             }
             // the owner of the top degree: r_{N-1} (A) or psi_{N-2} (B); zero elsewhere
             tops[p] = l == lt ? (A ? rt : ((PSI && L.psi) ? vt : fma(L.m, vt, -(rt * L.ibeta)))) : 0.0;
-            if (PSI && A) {  // u_{N-1}: the wall sum's remainder where the recursion has lost more
-                double ab[1][E], q[E], su = 0.0, sa = 0.0, lo = 0.0;
+            if (PSI && A && __any(rest)) {  // u_{N-1}: the wall sum's remainder
+                double su = 0.0;
 #pragma unroll
-                for (int i = 0; i < E; ++i) {
-                    const int k = k0 + 2 * i;
-                    const bool in = k < N - 1;
-                    if (piv) ab[0][i] = k == N - 1 ? fabs(L.m * (i > 0 ? e[p][i > 0 ? i - 1 : 0] : below)) * tau_lo(k) : 0.0;
-                    else ab[0][i] = in ? fabs(e[p][i]) : 0.0;
-                    su += in ? uu[i] : 0.0;
-                    sa += in ? fabs(uu[i]) : 0.0;
-                    if (k == N - 1) lo = fabs(e1[p][PSI ? i : 0]);
-                }
-                if (!piv) tau_scan_up<G, E, 1>(a, ab, q, l);
+                for (int i = 0; i < E; ++i) su += k0 + 2 * i < N - 1 ? uu[i] : 0.0;
                 su = lanes_sum<G>(su);
-                sa = lanes_sum<G>(sa);
 #pragma unroll
-                for (int i = 0; i < E; ++i)
-                    if (k0 + 2 * i == N - 1 && L.psi && (ab[0][i] + lo) * fabs(L.beta * L.ial) > sa + fabs(w[p]))
-                        uu[i] = w[p] - su;
+                for (int i = 0; i < E; ++i) uu[i] = rest && k0 + 2 * i == N - 1 ? w[p] - su : uu[i];
             }
 #pragma unroll
             for (int i = 0; i < E; ++i) r[i][p] = uu[i];  // beyond N - 1 a, e and r are zero
