@@ -31,7 +31,7 @@ enum Channel3Var : int { kC3P = 0, kC3B = 1, kC3UX = 2, kC3UY = 3, kC3UZ = 4 };
 
 // kernel variants picked by the autotuner at creation; every variant gives the same bits
 struct Chan3Tuning {
-    int solve = 0;  // k3_tau_solve workgroup: 0 one wave, 1 four
+    int solve = 0;  // k3_tau_solve workgroup: 0 one pair of waves, 1 two pairs
     int zbwd = 0;   // k3_zbwd mode tile: 0 the type's default (32 FP32 / 16 FP64), 1 16 modes (FP32 only)
 };
 

@@ -73,7 +73,7 @@ class ChannelSolver {
     TauSys tau_sys(double c) const;
     bool any_sign() const;  // a negative diffusivity
     template <typename T> TauArgs<T> solve_args() const;
-    int solve_wgs() const;  // workgroups (waves) of the solve kernel
+    int solve_wgs() const;  // workgroups (pairs of waves) of the solve kernel
     void advance_clock();
     template <typename T> void rhs_t(const void* b, const void* ux, const void* uz, void* F0, void* F1, void* F2);
     template <typename T> void lx_t(int s);

@@ -774,9 +774,9 @@ void zgetrf_batched(Context* c, void* A, int n, int nmodes, int* ipiv, int* info
         hipLaunchKernelGGL((k_zgetrf<NT, RPT>), dim3((unsigned)nmodes), dim3(NT), 0, c->stream,
                            static_cast<double2*>(A), n, ipiv, info.as<int>());
     };
-    // one panel row per thread while a workgroup has the threads, then two and three (the 16
-    // columns of a row are 64 registers of the 256 that 512 threads leave each); above, the
-    // panel stays in memory
+    // one panel row per thread while a workgroup has the threads, then two (the 16 columns of a
+    // row are 64 registers of the 256 that 512 threads leave each); above, the panel stays in
+    // memory
     if (n <= 128) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 1>{});
     else if (n <= 256) launch(std::integral_constant<int, 256>{}, std::integral_constant<int, 1>{});
     else if (n <= 512) launch(std::integral_constant<int, 512>{}, std::integral_constant<int, 1>{});
