@@ -44,3 +44,30 @@ def test_batched_lu_ties(gpu, oracle):
     batched_factor_(s)
     assert np.array_equal(s.pivots.cpu().numpy(), ipiv_ref)
     assert np.array_equal(s.A.cpu().numpy(), LU_ref)
+
+
+@pytest.mark.parametrize("n", [60, 129, 263, 400])
+def test_batched_lu_backward_error(gpu, oracle, n):
+    """P A - L U in long double, over |A|: no larger than the oracle's, which updates the trailing matrix term by
+    term (mean of four matrices)."""
+    from tarang_amd.matsolvers import batched_factor_
+    print(f"batched LU backward error n={n}", flush=True)
+    r = np.random.default_rng(n)
+    A = (r.standard_normal((n, n, 4)) + 1j * r.standard_normal((n, n, 4))) / np.sqrt(n) + 0.5 * np.eye(n)[:, :, None]
+    ref, piv, _ = oracle.batched_lu_factor(A)
+    s = lu_on_device(gpu, A)
+    batched_factor_(s)
+    assert np.array_equal(s.pivots.cpu().numpy(), piv)
+    got = s.A.cpu().numpy()
+
+    def backward(LU, m):
+        P = np.arange(n)
+        for k, p in enumerate(piv[:, m]):
+            P[[k, p - 1]] = P[[p - 1, k]]
+        LU = LU[:, :, m].astype(np.clongdouble)
+        R = A[P, :, m] - (np.tril(LU, -1) + np.eye(n)) @ np.triu(LU)
+        return np.linalg.norm(R.astype(complex)) / np.linalg.norm(A[:, :, m])
+
+    a, b = (np.mean([backward(x, m) for m in range(4)]) for x in (got, ref))
+    print(f"  backward error {a:.2e}, oracle {b:.2e}", flush=True)
+    assert a <= b
