@@ -334,7 +334,7 @@ void cheb_deriv(Context* c, const void* in, void* out, int ndim, const int* shap
 // An exactly zero pivot column is recorded in info (first one, 1-based) and skipped, as
 // LAPACK does.
 // Bound: the chain of a column (two barriers, the reduction, a reciprocal: 5700 clocks with 512
-// threads), half of the 1280 us of 129 matrices of n = 263; the products take a third, at 0.4 of the
+// threads), half of the 1260 us of 129 matrices of n = 263; the products take a third, at 0.4 of the
 // FP64 rate of their CU.  Before, panel and products from memory, thread by thread: 2965 us.
 // Whole calls: 1031 x 64 36 against 73 ms, 400 x 60 2.7 against 6.3 ms, 40 x 9 139 against 226 us.
 // ===========================================================================
